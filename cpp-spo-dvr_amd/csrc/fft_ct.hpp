@@ -147,6 +147,12 @@ __device__ __forceinline__ cx<T> mul_unit_root(cx<T> a, int sign) {
   } else if constexpr (sizeof(T) == 8) {
     constexpr CS w = unit_root(m, R);
     return a * cx<T>{T(w.c), T(sign) * T(w.s)};
+  } else if constexpr (R == 9) {
+    // FP32: the constant as hi + lo (mul_hilo); the four twiddles of a 9-point butterfly are few enough for it
+    constexpr CS w = unit_root(m, R);
+    constexpr float c = static_cast<float>(w.c), s = static_cast<float>(w.s);
+    constexpr float c_lo = static_cast<float>(w.c - c), s_lo = static_cast<float>(w.s - s);
+    return mul_hilo(cx<T>{c, T(sign) * s}, cx<T>{c_lo, T(sign) * s_lo}, a);
   } else {
     // FP32: a pair of floats of unit modulus (unit_f32), so that the twiddle does not scale its modes at every
     // transform
@@ -222,10 +228,16 @@ __device__ __forceinline__ void rdft(cx<T>* v, int sign) {
     dft<R, T>(v, sign);
   } else if constexpr (R == 6) {
     rdft_composite<3, 2, T>(v, sign);
+  } else if constexpr (R == 9) {
+    rdft_composite<3, 3, T>(v, sign);
   } else if constexpr (R == 10) {
     rdft_composite<5, 2, T>(v, sign);
   } else if constexpr (R == 12) {
     rdft_composite<4, 3, T>(v, sign);
+  } else if constexpr (R == 14) {
+    rdft_composite<7, 2, T>(v, sign);
+  } else if constexpr (R == 15) {
+    rdft_composite<5, 3, T>(v, sign);
   } else if constexpr (R == 16) {
     rdft_composite<4, 4, T>(v, sign);
   }

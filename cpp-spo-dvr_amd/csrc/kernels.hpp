@@ -343,7 +343,7 @@ __global__ void bk_scattering_kernel(const cx<T>* psi, Shape s, int iz_ana, int 
 }
 
 // The initial state from the specular wave at the fixed analysis surface (src/analysis/balint_kurti.cpp:74-82).
-__global__ void bk_specular_kernel(const cx<double>* spec, int nr, int iz_sp, int n_v, int n_states, int initial,
+__global__ inline void bk_specular_kernel(const cx<double>* spec, int nr, int iz_sp, int n_v, int n_states, int initial,
                                    const double* phi_in, double dr, cx<double>* bk) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= n_v) return;
@@ -353,7 +353,7 @@ __global__ void bk_specular_kernel(const cx<double>* spec, int nr, int iz_sp, in
 }
 
 // sums(k, ien) += c(k) exp(i E_ien t) dtAna, FP64 (src/analysis/s_matrix.cpp:49-56).
-__global__ void s_accumulate_kernel(cx<double>* sums, const cx<double>* bk, int n, int n_e, const double* energies,
+__global__ inline void s_accumulate_kernel(cx<double>* sums, const cx<double>* bk, int n, int n_e, const double* energies,
                                     double t, double dt_ana) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (long)n * n_e) return;
@@ -366,7 +366,7 @@ __global__ void s_accumulate_kernel(cx<double>* sums, const cx<double>* bk, int 
 
 // ---------------------------------------------------------------------------------------------------------------
 // Wave-packet utilities.
-__global__ void zero_kernel(cx<double>* p, long n) {
+__global__ inline void zero_kernel(cx<double>* p, long n) {
   const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k < n) p[k] = cx<double>{0.0, 0.0};
 }
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(256) void energy_resolved_kernel(const cx<T>* psi, 
 }
 
 // The same for the specular wave: sums[ien][k] += (spec[k] phase[ien]) dtAna over its n values (ir, iz).
-__global__ __launch_bounds__(256) void energy_resolved_specular_kernel(const cx<double>* spec, int n, int n_energies,
+__global__ inline __launch_bounds__(256) void energy_resolved_specular_kernel(const cx<double>* spec, int n, int n_energies,
                                                                        const cx<double>* phase, double dt,
                                                                        cx<double>* sums) {
   const int k = blockIdx.x * 256 + threadIdx.x;

@@ -11,18 +11,6 @@
 
 namespace spo_dev {
 
-// T_Zr with register-resident Stockham passes: NR = A1 * A2 and NZ = B1 * B2, two radix passes per axis, each pass
-// a set of whole butterflies per thread with one LDS exchange between passes. The first r pass reads its
-// butterflies straight from HBM and the last inverse r pass writes straight to HBM; the last forward Z pass, the
-// factor exp(-i (T_Z + T_r) dt) (FFT scales folded in) and the first inverse Z pass run on the same registers
-// (the inverse runs its radices in reverse order, so its first pass takes exactly the elements the forward pass
-// left in each thread). Seven passes, six LDS round trips, versus a tile in and out of LDS around every stage.
-//
-// Stockham positions for N = R1 * R2: pass 1 (radix R1) takes x[j + r R2] (j < R2) and writes j R1 + r; pass 2
-// (radix R2) takes j + r R1 (j < R1), twiddles by W_N^{r j} and writes back to the same places, in natural order.
-// Plane in LDS: row iz at iz * (NR + 1) (complex64: followed by the NR + NZ twiddles). The HBM passes (1 and 7) run lanes along j so that 16 lanes touch
-// consecutive addresses; with A1 odd, pass 1's LDS writes (stride A1) also spread over the banks. Passes 2 and 6
-// run lanes along iz (stride NR + 1, odd) and the Z passes along kr (stride 1).
 template <int NBUT, int THREADS>
 constexpr int per_thread() {
   return (NBUT + THREADS - 1) / THREADS;
@@ -55,13 +43,6 @@ constexpr bool zr_twiddles_in_lds() {
   return sizeof(T) == 4;
 }
 
-// LDS bytes of zr_reg_kernel (complex64: the twiddles and their remainders behind the plane).
-template <typename T>
-inline std::size_t zr_reg_lds(int nz, int nr) {
-  return std::size_t(nz) * (nr + 1) * sizeof(cx<T>) +
-         (zr_twiddles_in_lds<T>() ? std::size_t(nz + nr) * 2 * sizeof(cx<T>) : 0);
-}
-
 // twiddle() with the complex64 remainders already formed: lo[k * LS] = eps_k w_k (the part of the twiddle that
 // restores its modulus), applied through mul_hilo. FP64 passes no lo.
 template <typename T, int R, bool SKIP_ZERO = true, int TS = 1, int LS = 1>
@@ -80,210 +61,6 @@ __device__ __forceinline__ void twiddle_lo(cx<T>* v, const cx<T>* table, const c
     } else {
       if (sign > 0) w = conj(w);
       v[r] = v[r] * w;
-    }
-  }
-}
-
-// eps_z, eps_r: the complex64 twiddle tables' modulus corrections (twiddle()); factor_lo: the factor's FP32
-// remainders (mul_hilo). Unused in FP64.
-// row >= 0: psi is only read, and Z row `row` of each transformed plane (NR values) goes to row_out[plane * NR + ir]
-// (the inverse r passes run for that row alone); row < 0: psi is transformed in place and row_out is unused.
-template <typename T, int NZ, int NR, int A1, int A2, int B1, int B2, int THREADS>
-__global__ __launch_bounds__(THREADS) void zr_reg_kernel(cx<T>* psi, const cx<T>* table_z, const cx<T>* table_r,
-                                                         const cx<T>* factor, const T* eps_z, const T* eps_r,
-                                                         const cx<T>* factor_lo, cx<T>* row_out, int row) {
-  static_assert(A1 * A2 == NR && B1 * B2 == NZ, "zr_reg_kernel: radices must multiply to the lengths");
-  extern __shared__ unsigned char smem_raw[];
-  cx<T>* t = reinterpret_cast<cx<T>*>(smem_raw);
-  constexpr int P = NZ * NR;
-  constexpr int LD = NR + 1;
-  cx<T>* plane = psi + static_cast<long>(blockIdx.x) * P;
-  const int tid = threadIdx.x;
-  // complex64: the twiddle tables live in LDS behind the plane (lower latency than the cache for the in-pass
-  // twiddles); FP64 keeps them in the cache, where they do not compete with the plane for LDS bandwidth (measured
-  // on MI355X: 1.89 -> 1.73 ms and 3.85 -> 4.15 ms per time step respectively).
-  // complex64: each twiddle's remainder eps w is formed once here, so that the passes spend no products on it.
-  const cx<T>* lo_r = nullptr;
-  const cx<T>* lo_z = nullptr;
-  if constexpr (zr_twiddles_in_lds<T>()) {
-    cx<T>* tw_r = t + NZ * LD;
-    cx<T>* tw_z = tw_r + NR;
-    cx<T>* l_r = tw_z + NZ;
-    cx<T>* l_z = l_r + NR;
-    for (int e = tid; e < NR; e += THREADS) {
-      const cx<T> w = table_r[e];
-      const T k = eps_r[e];
-      tw_r[e] = w;
-      l_r[e] = {k * w.x, k * w.y};
-    }
-    for (int e = tid; e < NZ; e += THREADS) {
-      const cx<T> w = table_z[e];
-      const T k = eps_z[e];
-      tw_z[e] = w;
-      l_z[e] = {k * w.x, k * w.y};
-    }
-    table_r = tw_r;
-    table_z = tw_z;
-    lo_r = l_r;
-    lo_z = l_z;
-  }
-
-  // Pass 1, r forward, radix A1: butterfly (iz, j < A2) from HBM.
-  {
-    constexpr int N = NZ * A2, Q = per_thread<N, THREADS>();
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int j = b % A2, iz = b / A2;
-      cx<T> v[A1];
-#pragma unroll
-      for (int r = 0; r < A1; ++r) v[r] = plane[iz * NR + j + r * A2];
-      rdft<A1, T>(v, -1);
-#pragma unroll
-      for (int r = 0; r < A1; ++r) t[iz * LD + j * A1 + r] = v[r];
-    }
-  }
-  __syncthreads();
-  // Pass 2, r forward, radix A2, in place: butterfly (iz, j < A1), lanes along iz (row stride NR + 1).
-  {
-    constexpr int N = NZ * A1, Q = per_thread<N, THREADS>();
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int iz = b % NZ, j = b / NZ;
-      cx<T> v[A2];
-#pragma unroll
-      for (int r = 0; r < A2; ++r) v[r] = t[iz * LD + j + r * A1];
-      twiddle_lo<T, A2>(v, table_r, lo_r, j, -1);
-      rdft<A2, T>(v, -1);
-#pragma unroll
-      for (int r = 0; r < A2; ++r) t[iz * LD + j + r * A1] = v[r];
-    }
-  }
-  __syncthreads();
-  // Pass 3, Z forward, radix B1: butterfly (kr, j < B2); reads all, then writes all.
-  {
-    constexpr int N = NR * B2, Q = per_thread<N, THREADS>();
-    cx<T> v[Q][B1];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int kr = b % NR, j = b / NR;
-#pragma unroll
-      for (int r = 0; r < B1; ++r) v[q][r] = t[(j + r * B2) * LD + kr];
-      rdft<B1, T>(v[q], -1);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int kr = b % NR, j = b / NR;
-#pragma unroll
-      for (int r = 0; r < B1; ++r) t[(j * B1 + r) * LD + kr] = v[q][r];
-    }
-  }
-  __syncthreads();
-  // Pass 4, Z forward radix B2 (twiddled), x factor, Z inverse radix B2: butterfly (kr, j < B1).
-  {
-    constexpr int N = NR * B1, Q = per_thread<N, THREADS>();
-    cx<T> v[Q][B2];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int kr = b % NR, j = b / NR;
-#pragma unroll
-      for (int r = 0; r < B2; ++r) v[q][r] = t[(j + r * B1) * LD + kr];
-      twiddle_lo<T, B2>(v[q], table_z, lo_z, j, -1);
-      rdft<B2, T>(v[q], -1);
-#pragma unroll
-      for (int r = 0; r < B2; ++r) {
-        const int f = (j + r * B1) * NR + kr;
-        v[q][r] = mul_factor(factor[f], v[q][r], factor_lo, f);
-      }
-      rdft<B2, T>(v[q], +1);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int kr = b % NR, j = b / NR;
-#pragma unroll
-      for (int r = 0; r < B2; ++r) t[(j * B2 + r) * LD + kr] = v[q][r];
-    }
-  }
-  __syncthreads();
-  // Pass 5, Z inverse, radix B1, in place: butterfly (kr, j < B2).
-  {
-    constexpr int N = NR * B2, Q = per_thread<N, THREADS>();
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int kr = b % NR, j = b / NR;
-      cx<T> v[B1];
-#pragma unroll
-      for (int r = 0; r < B1; ++r) v[r] = t[(j + r * B2) * LD + kr];
-      twiddle_lo<T, B1>(v, table_z, lo_z, j, +1);
-      rdft<B1, T>(v, +1);
-#pragma unroll
-      for (int r = 0; r < B1; ++r) t[(j + r * B2) * LD + kr] = v[r];
-    }
-  }
-  __syncthreads();
-  // Pass 6, r inverse, radix A2: butterfly (iz, j < A1), lanes along iz; reads all, then writes all.
-  {
-    constexpr int N = NZ * A1, Q = per_thread<N, THREADS>();
-    cx<T> v[Q][A2];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int iz = b % NZ, j = b / NZ;
-      if (row >= 0 && iz != row) continue;
-#pragma unroll
-      for (int r = 0; r < A2; ++r) v[q][r] = t[iz * LD + j + r * A1];
-      rdft<A2, T>(v[q], +1);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int iz = b % NZ, j = b / NZ;
-      if (row >= 0 && iz != row) continue;
-#pragma unroll
-      for (int r = 0; r < A2; ++r) t[iz * LD + j * A2 + r] = v[q][r];
-    }
-  }
-  __syncthreads();
-  // Pass 7, r inverse, radix A1 (twiddled): butterfly (iz, j < A2) to HBM.
-  {
-    constexpr int N = NZ * A2, Q = per_thread<N, THREADS>();
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int b = tid + q * THREADS;
-      if (N % THREADS != 0 && b >= N) break;
-      const int j = b % A2, iz = b / A2;
-      if (row >= 0 && iz != row) continue;
-      cx<T> v[A1];
-#pragma unroll
-      for (int r = 0; r < A1; ++r) v[r] = t[iz * LD + j + r * A2];
-      twiddle_lo<T, A1>(v, table_r, lo_r, j, +1);
-      rdft<A1, T>(v, +1);
-      if (row >= 0) {
-        cx<T>* out = row_out + static_cast<long>(blockIdx.x) * NR;
-#pragma unroll
-        for (int r = 0; r < A1; ++r) out[j + r * A2] = v[r];
-      } else {
-#pragma unroll
-        for (int r = 0; r < A1; ++r) plane[iz * NR + j + r * A2] = v[r];
-      }
     }
   }
 }
@@ -555,7 +332,7 @@ __global__ void densities_partial_kernel(const cx<T>* psi, Shape s, int chunk, d
   partial[izr + static_cast<long>(s.n_zr) * part] = acc;
 }
 
-__global__ void densities_sum_kernel(const double* partial, int n_zr, int parts, double* out) {
+__global__ inline void densities_sum_kernel(const double* partial, int n_zr, int parts, double* out) {
   const int izr = blockIdx.x * blockDim.x + threadIdx.x;
   if (izr >= n_zr) return;
   double acc = 0.0;

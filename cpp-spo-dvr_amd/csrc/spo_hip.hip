@@ -25,10 +25,13 @@
 #include "../../include/spo_hip.h"
 #include "kernels_ct.hpp"
 #include "kernels_mfma.hpp"
+#include "kernels_zr.hpp"
+#include "variants.hpp"
 #include "kernels_pes.hpp"
 #include "kernels_mlp.hpp"
 
 using spo_dev::cx;
+using spo_dev::Variant;
 
 namespace {
 
@@ -199,126 +202,6 @@ constexpr int kThreads = 256;
 
 void set_lds(const void* kernel, std::size_t bytes) {
   HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
-}
-
-// ---- instantiations of the compile-time-shaped kernels ---------------------------------------------------------
-// Phi lengths of the interaction kernel with the contractions on the vector units.
-#define SPO_PHI_LENGTHS(X) X(48) X(22) X(10) X(12) X(8) X(56)
-// T_Zr planes with register-resident passes (NZ, NR, A1, A2, B1, B2, threads): NR = A1 A2, NZ = B1 B2. Entries of
-// one shape that differ only in the thread count compute identically; the launch tuner picks among them.
-// Other factorisations of a shape (the radices of each axis) are further entries of that shape: they compute the same
-// transforms with their roundings in another order, and the launch tuner picks among them as among block sizes.
-#define SPO_ZR_REG_SHAPES(X)                                                                                 \
-  X(96, 48, 3, 16, 12, 8, 192) X(96, 48, 3, 16, 8, 12, 192) X(96, 48, 4, 12, 8, 12, 192)                      \
-  X(96, 48, 3, 16, 8, 12, 384) X(96, 48, 3, 16, 8, 12, 512) X(96, 48, 3, 16, 12, 8, 384)                       \
-  X(96, 48, 12, 4, 8, 12, 384)                                                                                 \
-  X(128, 32, 4, 8, 16, 8, 256) X(128, 32, 4, 8, 16, 8, 512) X(64, 16, 4, 4, 8, 8, 128) X(80, 16, 4, 4, 8, 10, 128) \
-  X(176, 56, 7, 8, 11, 16, 256) X(176, 56, 7, 8, 11, 16, 512) X(96, 32, 4, 8, 8, 12, 256)                      \
-  X(96, 32, 4, 8, 8, 12, 512)
-// Interaction with the theta contractions on MFMA (phi length, wavefronts, phi radices R1 x R2 of the fused phi
-// step); the staged-FFT variant is instantiated with 8 wavefronts.
-#define SPO_MFMA_SHAPES(X)                                                                                   \
-  X(48, 8, 12, 4) X(48, 4, 12, 4) X(48, 16, 12, 4) X(22, 8, 11, 2) X(12, 8, 4, 3) X(10, 8, 5, 2)             \
-  X(8, 8, 4, 2) X(56, 8, 8, 7) X(56, 4, 8, 7)
-// T_xy tiles with whole-line DFTs in registers (NX = NY a single radix; C izr per tile, C * NX threads).
-#define SPO_XY_REG_SHAPES(X) X(16, 16, 32) X(16, 16, 16) X(16, 16, 8) X(8, 8, 32) X(8, 8, 16) X(4, 4, 64) X(4, 4, 32)
-// The buffer-addressed interaction kernel (phi length, wavefronts, phi radices): the MFMA shapes, the phi steps of
-// the reduced-JMax batch members (28 and 40 points) and two more factorisations of the 48-point step (16 x 3,
-// 8 x 6) for the launch tuner.
-#define SPO_BUF_SHAPES(X) SPO_MFMA_SHAPES(X) X(28, 8, 7, 4) X(40, 8, 10, 4) X(48, 8, 16, 3) X(48, 8, 8, 6)
-
-// A launch variant of a kernel family: the kernel, its block size, its tile parameter (T_xy: izr per tile;
-// interaction: wavefronts) and its LDS bytes.
-struct Variant {
-  const void* fn;
-  int threads;
-  int param;
-  std::size_t lds;
-};
-
-template <typename T>
-std::vector<Variant> zr_reg_variants(int nz, int nr) {
-  std::vector<Variant> out;
-#define X(A, B, A1, A2, B1, B2, TH)                                                                        \
-  if (nz == A && nr == B)                                                                                  \
-    out.push_back({reinterpret_cast<const void*>(spo_dev::zr_reg_kernel<T, A, B, A1, A2, B1, B2, TH>), TH, \
-                   TH, spo_dev::zr_reg_lds<T>(A, B)});
-  SPO_ZR_REG_SHAPES(X)
-#undef X
-  // Default (first) variant, as measured on MI355X at NZ 96 x NR 48: FP64 planes run best with the largest thread
-  // count (512 threads: 3.42 ms per time step; 384: 3.44; 192: 4.2-4.5), complex64 planes with the smallest one, and
-  // among those with the Z radices 12 x 8 (1.88 ms; 8 x 12: 1.92; r radices 4 x 12: 1.91; 6 x 8, 12 x 4 and the Z
-  // radices 16 x 6 or 6 x 16: 1.98-2.15). Ties keep the order of the shape list.
-  std::stable_sort(out.begin(), out.end(), [](const Variant& a, const Variant& b) {
-    return sizeof(T) == 8 ? a.threads > b.threads : a.threads < b.threads;
-  });
-  return out;
-}
-
-template <typename T>
-std::vector<Variant> xy_reg_variants(int nx, int ny) {
-  std::vector<Variant> out;
-  // FP64 tiles of 16 izr at 16 x 16 go through LDS in halves (xy_reg_kernel SPLIT): 35 KB instead of 70 KB.
-#define X(A, B, CC)                                                                                          \
-  if (nx == A && ny == B) {                                                                                  \
-    constexpr bool split = sizeof(T) == 8 && A == 16 && CC == 16;                                            \
-    out.push_back({reinterpret_cast<const void*>(spo_dev::xy_reg_kernel<T, A, B, CC, split>), CC * A, CC,    \
-                   spo_dev::xy_reg_lds<T>(A, B, CC, split)});                                               \
-  }
-  SPO_XY_REG_SHAPES(X)
-#undef X
-  // Default (first) variant, as measured on MI355X: the widest tile in both precisions. FP64 at 16 x 16: tiles of
-  // 32 izr 3.04 ms per time step, of 16 (through LDS in halves) 3.12, of 8 3.43; at 8 x 8: 32 izr 0.112, 16 izr
-  // 0.115. Complex64 at 16 x 16: 32 izr 1.76, 16 izr 1.90, 8 izr 2.58.
-  std::stable_sort(out.begin(), out.end(), [](const Variant& a, const Variant& b) { return a.param > b.param; });
-  return out;
-}
-
-// fused: the phi step in three register passes (phi_step_fused) rather than the staged LDS FFTs (8 wavefronts).
-template <typename T>
-std::vector<Variant> interaction_mfma_variants(int nphi, int n_theta, bool fused) {
-  constexpr int NT = 1;  // 8 columns: one 128-byte line of an irot row in FP64 (two complex64 tiles ran slower)
-  std::vector<Variant> out;
-  const std::size_t lds = spo_dev::interaction_mfma_lds<T>(8 * NT, n_theta, nphi, fused);
-#define X(A, W, R1, R2)                                                                                      \
-  if (nphi == A && (fused || W == 8))                                                                        \
-    out.push_back({fused ? reinterpret_cast<const void*>(spo_dev::interaction_mfma_kernel<T, A, NT, W, R1, R2>) \
-                         : reinterpret_cast<const void*>(spo_dev::interaction_mfma_kernel<T, A, NT, W>),     \
-                   64 * W, W, lds});
-  SPO_MFMA_SHAPES(X)
-#undef X
-  return out;
-}
-
-// The buffer-addressed interaction kernel: every MFMA shape with at most 8 mJ blocks per wavefront; bf16x3: the
-// complex64 split-BF16x3 contraction variant (instantiated for the 48-point phi step).
-template <typename T>
-std::vector<Variant> interaction_buf_variants(int nphi, int n_theta, int n_blocks, bool bf16x3) {
-  std::vector<Variant> out;
-  const std::size_t lds = spo_dev::interaction_buf_lds<T>(n_theta, nphi);
-  if (bf16x3) {
-    if constexpr (sizeof(T) == 4) {
-      if (nphi == 48 && n_blocks <= 64)
-        out.push_back({reinterpret_cast<const void*>(spo_dev::interaction_buf_kernel<T, 48, 8, 12, 4, true>), 512,
-                       8, lds});
-    }
-    return out;
-  }
-#define X(A, W, R1, R2)                                                                                         \
-  if (nphi == A && n_blocks <= 8 * W)                                                                           \
-    out.push_back({reinterpret_cast<const void*>(spo_dev::interaction_buf_kernel<T, A, W, R1, R2>), 64 * W, W, lds});
-  SPO_BUF_SHAPES(X)
-#undef X
-  return out;
-}
-
-template <typename T>
-const void* interaction_ct_symbol(int nphi) {
-#define X(A) \
-  if (nphi == A) return reinterpret_cast<const void*>(spo_dev::interaction_ct_kernel<T, A, kThreads>);
-  SPO_PHI_LENGTHS(X)
-#undef X
-  return nullptr;
 }
 
 // Launch through the symbol with a packed argument list (hipLaunchKernel), so one call covers every instantiation.
@@ -531,6 +414,10 @@ struct State final : spo_hip_backend {
   const void* v_fn = nullptr;
   bool zr_fused = false;
 
+  // The T_Zr factors in the order of zr_inplace_kernel's places (order_zr_factors, for the variant in use).
+  Buffer zr_full_p, zr_half_p, zr_full_p_lo, zr_half_p_lo;
+  void order_zr_factors(const std::vector<double>& full, const std::vector<double>& half, const spo_dev::ZrShape& order);
+
   Buffer ana_row;  // the analysis row of the scattering wave at the analysis time (merged half steps)
 
   void run_zr(const Variant& v, bool half, cx<T>* row_out = nullptr, int row = -1);
@@ -570,13 +457,32 @@ void State<T>::run_zr(const Variant& v, bool half, cx<T>* row_out, int row) {
   cx<T>* ps = psi.as<cx<T>>();
   const cx<T>* tz = plan_z->tw();
   const cx<T>* tr = plan_r->tw();
-  const cx<T>* zr = (half ? zr_half : zr_full).as<cx<T>>();
   const T* ez = plan_z->tw_eps();
   const T* er = plan_r->tw_eps();
-  const cx<T>* fl = (half ? zr_half_lo : zr_full_lo).as<cx<T>>();
-  void* args[] = {&ps, const_cast<cx<T>**>(&tz), const_cast<cx<T>**>(&tr), const_cast<cx<T>**>(&zr),
+  spo_dev::ZrShape shape = v.zr;
+  const cx<T>* zr = (half ? zr_half_p : zr_full_p).as<cx<T>>();
+  const cx<T>* fl = (half ? zr_half_p_lo : zr_full_p_lo).as<cx<T>>();
+  void* args[] = {&ps, &shape, const_cast<cx<T>**>(&tz), const_cast<cx<T>**>(&tr), const_cast<cx<T>**>(&zr),
                   const_cast<T**>(&ez), const_cast<T**>(&er), const_cast<cx<T>**>(&fl), &row_out, &row};
   launch(v.fn, s.n_rot * s.n_xy, v.threads, v.lds, stream, args);
+}
+
+template <typename T>
+void State<T>::order_zr_factors(const std::vector<double>& full, const std::vector<double>& half,
+                                const spo_dev::ZrShape& order) {
+  std::vector<double> f(full.size()), h(half.size());
+  for (int iz = 0; iz < s.nz; ++iz)
+    for (int ir = 0; ir < s.nr; ++ir) {
+      const std::size_t to = 2 * (ir + std::size_t(s.nr) * iz), from = 2 * spo_dev::zr_factor_order(order, iz, ir);
+      for (int c = 0; c < 2; ++c) {
+        f[to + c] = full[from + c];
+        h[to + c] = half[from + c];
+      }
+    }
+  zr_full_p = upload_complex<T>(f.data(), s.n_zr);
+  zr_full_p_lo = factor_lo<T>(f.data(), s.n_zr);
+  zr_half_p = upload_complex<T>(h.data(), s.n_zr);
+  zr_half_p_lo = factor_lo<T>(h.data(), s.n_zr);
 }
 
 template <typename T>
@@ -1013,12 +919,15 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
     for (double& x : v) x = x * f1 * f2;
     return v;
   };
+  std::vector<double> zr_full_values, zr_half_values;
   {
     const auto zf = fold(t->zr_full, s.n_zr, zr_f, zr_b), zh = fold(t->zr_half, s.n_zr, zr_f, zr_b);
     b->zr_full = upload_complex<T>(zf.data(), s.n_zr);
     b->zr_full_lo = factor_lo<T>(zf.data(), s.n_zr);
     b->zr_half = upload_complex<T>(zh.data(), s.n_zr);
     b->zr_half_lo = factor_lo<T>(zh.data(), s.n_zr);
+    zr_full_values = zf;
+    zr_half_values = zh;
     const auto sf = fold(t->specular_full, std::size_t(s.nr) * s.nzsp, zr_f, sp_b);
     const auto sh = fold(t->specular_half, std::size_t(s.nr) * s.nzsp, zr_f, sp_b);
     b->spec_full = upload(sf.data(), sf.size() * sizeof(double));
@@ -1124,17 +1033,19 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
   b->plan_x_d = std::make_unique<DevicePlan<double>>(s.nx);
   b->plan_y_d = std::make_unique<DevicePlan<double>>(s.ny);
   const std::size_t lds_limit = static_cast<std::size_t>(b->max_lds);
-  // T_Zr: the register-pass kernel (padded rows) if instantiated and it fits, else the run-time one, else lines.
-  if (spo_dev::zr_reg_lds<T>(s.nz, s.nr) <= lds_limit) b->zr_variants = zr_reg_variants<T>(s.nz, s.nr);
+  // T_Zr: the register-pass kernel where the axes are products of two radices and the plane fits in LDS, else the
+  // run-time engine on the plane, else lines.
+  if (spo_dev::zr_plane_lds<T>(s.nz, s.nr) <= lds_limit) b->zr_variants = spo_dev::zr_variants<T>(s.nz, s.nr);
   if (!b->zr_variants.empty()) {
     for (const Variant& v : b->zr_variants) set_lds(v.fn, v.lds);
+    b->order_zr_factors(zr_full_values, zr_half_values, b->zr_variants[0].zr);
   } else if (std::size_t(s.n_zr) * cT <= lds_limit) {
     b->zr_fused = true;
     b->zr_lds = std::size_t(s.n_zr) * cT;
     set_lds(reinterpret_cast<const void*>(spo_dev::zr_plane_kernel<T>), b->zr_lds);
   }
   // T_xy.
-  for (const Variant& v : xy_reg_variants<T>(s.nx, s.ny))
+  for (const Variant& v : spo_dev::xy_reg_variants<T>(s.nx, s.ny))
     if (v.lds <= lds_limit) b->xy_variants.push_back(v);
   if (!b->xy_variants.empty()) {
     for (const Variant& v : b->xy_variants) set_lds(v.fn, v.lds);
@@ -1145,7 +1056,7 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
     set_lds(reinterpret_cast<const void*>(spo_dev::xy_kernel<T>), b->xy_lds);
   }
   // Interaction tile: the largest power of two of columns (at most 32) whose LDS fits in 80 KiB (two per CU).
-  b->v_fn = s.n_theta <= spo_dev::kMaxTheta ? interaction_ct_symbol<T>(s.n_phi) : nullptr;
+  b->v_fn = s.n_theta <= spo_dev::kMaxTheta ? spo_dev::interaction_ct_symbol<T>(s.n_phi) : nullptr;
   auto v_bytes = [&](int c) {
     return b->v_fn ? spo_dev::interaction_ct_lds<T>(c, s.n_theta, s.n_phi, b->legendre_size)
                    : std::size_t(c) * (s.n_rot + s.n_tp) * cT;
@@ -1174,11 +1085,11 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
       throw Status(SPO_HIP_E_ARGUMENT, "SPO_HIP_CONTRACTION must be fp32 or bf16x3");
     const bool bf16x3 = sizeof(T) == 4 && contraction && std::string(contraction) == "bf16x3";
     std::vector<Variant> variants;
-    for (const Variant& v : interaction_mfma_variants<T>(s.n_phi, s.n_theta, fused))
+    for (const Variant& v : spo_dev::interaction_mfma_variants<T>(s.n_phi, s.n_theta, fused))
       if (v.lds <= lds_limit) variants.push_back(v);
     // phi lengths with a buffer-kernel instantiation only (the reduced-JMax batch members' 28 and 40 points)
     const bool buf_candidate =
-        choice == "buf" && !interaction_buf_variants<T>(s.n_phi, s.n_theta, s.n_blocks, bf16x3).empty();
+        choice == "buf" && !spo_dev::interaction_buf_variants<T>(s.n_phi, s.n_theta, s.n_blocks, bf16x3).empty();
     if ((!variants.empty() || buf_candidate) && choice != "lds") {
       const int n_tt = (s.n_theta + 15) / 16, k_bwd = (s.n_theta + 3) / 4;
       std::vector<int> fo(s.n_blocks), bo(s.n_blocks);
@@ -1233,7 +1144,7 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
       if (choice == "buf" && s.n_theta <= 16 && max_nb <= 16 &&
           std::size_t(s.n_zr) * s.n_rot * cT < (std::size_t(1) << 31)) {
         std::vector<Variant> buf;
-        for (const Variant& v : interaction_buf_variants<T>(s.n_phi, s.n_theta, s.n_blocks, bf16x3))
+        for (const Variant& v : spo_dev::interaction_buf_variants<T>(s.n_phi, s.n_theta, s.n_blocks, bf16x3))
           if (v.lds <= lds_limit) buf.push_back(v);
         if (bf16x3 && buf.empty())
           throw Status(SPO_HIP_E_NOT_SUPPORTED, "SPO_HIP_CONTRACTION=bf16x3: instantiated for the 48-point phi step only");
@@ -1323,6 +1234,8 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
   }
   HIP_CHECK(hipStreamSynchronize(b->stream));
   b->tune();
+  if (b->zr_pick != 0)
+    b->order_zr_factors(zr_full_values, zr_half_values, b->zr_variants[b->zr_pick].zr);
   return b;
 }
 

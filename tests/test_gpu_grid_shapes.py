@@ -1,0 +1,58 @@
+"""Grids of every kind of shape against the CPU oracle on one full T block: the radices of the T_Zr passes, the (x, y)
+line lengths and the angular bases for which the kernels choose between their paths. FP64 to the parity bar of
+test_gpu_parity.py (max |a - b| / max |a| < 1e-12), complex64 to single-precision rounding (< 1e-5)."""
+
+import os
+
+import numpy as np
+import pytest
+
+from tests import cases
+from tests.util import pseudo_random, relative_difference
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(nz, nr, nxy, jmax, **more):
+    """SMOKE_DAILIGHT on another grid of the same extent, its absorbers ending at the last grid points."""
+    dz, dr = 10.08 / (nz - 1), 4.5 / (nr - 1)
+    nzsp = 2 * nz
+    return dict(cases.SMOKE_DAILIGHT, Title=f"{nz} x {nr} x {nxy} x {nxy}, JMax {jmax}", nZ=nz, dZ=dz,
+                nR=nr, dR=dr, nX=nxy, nY=nxy, JMax=jmax, MJMax=more.pop("mjmax", jmax), nZSpecular=nzsp, ZOptEnd=-1.0 + dz * (nz - 1),
+                ROptEnd=0.8 + dr * (nr - 1), ZSpOptEnd=-1.0 + dz * (nzsp - 1), **more)
+
+
+def _check(name, params, seed, precisions=("fp64", "mixed"), blocks=((False, False),)):
+    import spodvr_amd
+    from oracle import oracle
+    path = cases.write_case(name, params)
+    cpu = oracle.run(path)
+    scattering, specular = pseudo_random(cpu.scattering_size, seed), pseudo_random(cpu.specular_size, seed + 1)
+    for half, kinetic_only in blocks:
+        cpu.set_wave(scattering, specular)
+        cpu.kinetic_and_potential(half, kinetic_only)
+        want = cpu.get_wave()
+        for precision in precisions:
+            print(f"{name} seed {seed} {precision} half {half} kinetic_only {kinetic_only}", flush=True)
+            os.environ["SPO_HIP_POTENTIAL"] = "host"
+            try:
+                gpu = spodvr_amd.Run(path, {"Precision": precision}, device="hip")
+            finally:
+                os.environ.pop("SPO_HIP_POTENTIAL", None)
+            gpu.set_wave(scattering, specular)
+            gpu.kinetic_and_potential(half, kinetic_only)
+            got = gpu.get_wave()
+            gpu.close()
+            ds, dp = (relative_difference(a, b) for a, b in zip(want, got))
+            print(f"  scattering {ds:.3e} specular {dp:.3e}", flush=True)
+            assert np.isfinite(got[0].view(float)).all()
+            assert ds < (1e-12 if precision == "fp64" else 1e-5) and dp < (1e-12 if precision == "fp64" else 1e-5)
+    cpu.close()
+
+
+# (NZ, NR): a prime radix alone (22 = 2 x 11), every radix up to 16 in each pass, axes of one radix and of two equal
+# ones, a length that is no product of two radices (the run-time engine), and a plane that fills a CU's LDS in FP64.
+@pytest.mark.parametrize("nz,nr", [(66, 12), (110, 14), (126, 22), (80, 30), (144, 18), (210, 20), (128, 56),
+                                   (112, 36), (160, 40), (192, 16), (264, 12), (132, 64)])
+def test_zr_plane_shapes(nz, nr):
+    _check(f"zr_{nz}_{nr}", _grid(nz, nr, 4, 2), 100 + nz + nr, blocks=((False, False), (True, True)))

@@ -243,6 +243,9 @@ __device__ __forceinline__ void rdft(cx<T>* v, int sign) {
   }
 }
 
+// The lengths rdft transforms.
+constexpr bool register_radix(int r) { return r >= 1 && r <= 16 && r != 13; }
+
 // ---- one stage, whole sequences per round ---------------------------------------------------------------------
 // Sequence s starts at (s % INNER) * IS + (s / INNER) * OS (INNER = 0: at s * IS); elements ES apart.
 template <int INNER, int IS, int OS, int ES>

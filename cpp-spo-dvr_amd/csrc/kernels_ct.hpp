@@ -74,11 +74,6 @@ __device__ __forceinline__ void twiddle_lo(cx<T>* v, const cx<T>* table, const c
 // SPLIT: each round trip goes through LDS in two halves of the y lines (rows iy < NY / 2, then the rest; four
 // barriers each), so that the tile takes half the LDS and twice as many workgroups fit on a CU. At least three
 // wavefronts per SIMD are asked for (FP64 at 16 x 16 needs 169 VGPRs otherwise, two wavefronts per SIMD).
-template <int N>
-constexpr bool single_radix() {
-  return is_radix(N);
-}
-
 // LDS bytes of xy_reg_kernel.
 template <typename T>
 constexpr std::size_t xy_reg_lds(int nx, int ny, int c, bool split) {
@@ -90,7 +85,7 @@ __global__ __launch_bounds__(C * NX) __attribute__((amdgpu_waves_per_eu(3))) voi
                                                          const cx<T>* shift_f, const cx<T>* shift_b, int needs_shift,
                                                          int apply_potential, const T* z_opt, const cx<T>* before,
                                                          const cx<T>* gas_step, XyLo<T> lo) {
-  static_assert(single_radix<NX>() && single_radix<NY>() && NX == NY, "xy_reg_kernel: one radix per axis, NX = NY");
+  static_assert(register_radix(NX) && NX == NY, "xy_reg_kernel: one radix per axis, NX = NY");
   static_assert(!SPLIT || NY % 2 == 0, "xy_reg_kernel: halves of the y lines");
   extern __shared__ unsigned char smem_raw[];
   cx<T>* tile = reinterpret_cast<cx<T>*>(smem_raw);

@@ -35,12 +35,14 @@ struct ZrShape {
   unsigned inv_a2, inv_nz, inv_nr;
 };
 
+// fast_div's multiplier for the divisor n.
+inline unsigned inverse_of(int n) { return n == 1 ? 0u : static_cast<unsigned>(((1ull << 32) + n - 1) / n); }
+
 __device__ __forceinline__ int fast_div(int x, int n, unsigned inv) {
   return n == 1 ? x : static_cast<int>(__umulhi(static_cast<unsigned>(x), inv));
 }
 
-// Radices of the run-time-shaped passes; f is called with the radix as a compile-time constant.
-constexpr bool zr_radix(int r) { return r >= 1 && r <= 16 && r != 13; }
+// Calls f with the radix as a compile-time constant.
 template <class F>
 __device__ __forceinline__ void with_radix(int r, F&& f) {
   switch (r) {

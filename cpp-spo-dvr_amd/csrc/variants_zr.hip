@@ -2,7 +2,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdint>
 
 #include "variants.hpp"
 
@@ -32,13 +31,12 @@ struct RadixPair {
 };
 RadixPair radix_pair(int n) {
   for (int low = 16; low >= 1; --low)
-    if (low * low <= n && n % low == 0 && zr_radix(low) && zr_radix(n / low)) return {low, n / low};
+    if (low * low <= n && n % low == 0 && register_radix(low) && register_radix(n / low)) return {low, n / low};
   return {0, 0};
 }
 
 ZrShape zr_shape(int nz, int nr, int a1, int a2, int b1, int b2) {
-  auto inverse = [](int n) { return static_cast<unsigned>(((std::uint64_t(1) << 32) + n - 1) / n); };
-  return {nz, nr, a1, a2, b1, b2, inverse(a2), inverse(nz), inverse(nr)};
+  return {nz, nr, a1, a2, b1, b2, inverse_of(a2), inverse_of(nz), inverse_of(nr)};
 }
 
 }  // namespace

@@ -56,3 +56,10 @@ def _check(name, params, seed, precisions=("fp64", "mixed"), blocks=((False, Fal
                                    (112, 36), (160, 40), (192, 16), (264, 12), (132, 64)])
 def test_zr_plane_shapes(nz, nr):
     _check(f"zr_{nz}_{nr}", _grid(nz, nr, 4, 2), 100 + nz + nr, blocks=((False, False), (True, True)))
+
+
+# Every (x, y) line length of the register kernel, with izr counts that leave a partial tile, and one beyond it.
+@pytest.mark.parametrize("nxy", [2, 6, 10, 12, 14, 18])
+@pytest.mark.parametrize("nz,nr", [(22, 10), (28, 12)])
+def test_xy_line_lengths(nxy, nz, nr):
+    _check(f"xy_{nxy}_{nz}_{nr}", _grid(nz, nr, nxy, 2), 200 + nxy + nz, blocks=((False, False), (True, True)))

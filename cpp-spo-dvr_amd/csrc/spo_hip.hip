@@ -1667,94 +1667,58 @@ int spo_hip_accumulate(spo_hip_backend* b, double time, const double* coefficien
 
 }  // extern "C"
 
-// The potential surrogate's device state: FP32 master parameters, gradient, Adam moments, and activation buffers
-// for `capacity` rows.
+// The potential surrogate's device state: FP32 master parameters, the hidden layers' bf16 fragments, Adam moments, what
+// a training pass leaves for the gradient (made at the first one), and the rows of a call (grown to the largest one so
+// far).
 struct spo_hip_mlp {
   int batch = 0;
-  long capacity = 0;
   int adam_step = 0;
-  Buffer params, grad, m, v;
-  Buffer x, t, y, dy, z1, a1, z2, a2, z3, a3, d1, d2;
+  Buffer params, frag, grad, m, v;
+  Buffer operands, values, errors;
+  spo_dev::MlpTape tape{};
+  Buffer x, t, y, losses;
+  long x_values = 0, t_values = 0, y_values = 0, loss_values = 0;
 };
 
 namespace {
 
-using spo_dev::kMlpWidth;
-
-void mlp_forward(spo_hip_mlp& n, long rows, const float* x) {
-  const float* p = n.params.as<float>();
-  const long cells = rows * kMlpWidth;
-  hipLaunchKernelGGL(spo_dev::mlp_input_kernel, dim3(blocks_for(cells, 256)), dim3(256), 0, nullptr, x, p, rows,
-                     n.z1.as<float>(), n.a1.as<float>());
-  const int tiles_j = kMlpWidth / 16;
-  const dim3 grid(static_cast<unsigned>(rows / 16 * tiles_j));
-  hipLaunchKernelGGL(spo_dev::mlp_gemm_kernel, grid, dim3(64), 0, nullptr, n.a1.as<float>(), long(kMlpWidth), 1L,
-                     p + spo_dev::kMlpW2, long(kMlpWidth), 1L, kMlpWidth, tiles_j, n.z2.as<float>(), long(kMlpWidth), 1,
-                     p + spo_dev::kMlpB2, n.a2.as<float>());
-  hipLaunchKernelGGL(spo_dev::mlp_gemm_kernel, grid, dim3(64), 0, nullptr, n.a2.as<float>(), long(kMlpWidth), 1L,
-                     p + spo_dev::kMlpW3, long(kMlpWidth), 1L, kMlpWidth, tiles_j, n.z3.as<float>(), long(kMlpWidth), 1,
-                     p + spo_dev::kMlpB3, n.a3.as<float>());
-  hipLaunchKernelGGL(spo_dev::mlp_output_kernel, dim3(blocks_for(rows, 256)), dim3(256), 0, nullptr, n.a3.as<float>(),
-                     p, rows, n.y.as<float>());
-  HIP_CHECK(hipGetLastError());
+// `b`, holding at least `count` floats; `have` is its size.
+float* at_least(Buffer& b, long& have, long count) {
+  if (have < count) {
+    have = 0;
+    b = Buffer();  // the old memory first
+    b = Buffer(std::size_t(count) * sizeof(float));
+    have = count;
+  }
+  return b.as<float>();
 }
 
-// The gradient of the mean squared error over `rows` rows into n.grad (after mlp_forward on the same rows).
-void mlp_backward(spo_hip_mlp& n, long rows, const float* x, const float* t, float* loss) {
-  const float* p = n.params.as<float>();
-  float* g = n.grad.as<float>();
-  const long cells = rows * kMlpWidth;
-  const int tiles = kMlpWidth / 16;
-  const long H = kMlpWidth;
-  hipLaunchKernelGGL(spo_dev::mlp_loss_kernel, dim3(1), dim3(256), 0, nullptr, n.y.as<float>(), t, rows,
-                     n.dy.as<float>(), loss);
-  hipLaunchKernelGGL(spo_dev::mlp_column_sum_kernel, dim3(kMlpWidth), dim3(256), 0, nullptr, n.a3.as<float>(), H,
-                     n.dy.as<float>(), rows, g + spo_dev::kMlpW4);
-  hipLaunchKernelGGL(spo_dev::mlp_column_sum_kernel, dim3(1), dim3(256), 0, nullptr, n.dy.as<float>(), 1L,
-                     static_cast<const float*>(nullptr), rows, g + spo_dev::kMlpB4);
-  float* dz3 = n.d2.as<float>();  // dZ3, then dA2 / dZ2 in d1, then dA1 / dZ1 in d2
-  hipLaunchKernelGGL(spo_dev::mlp_output_back_kernel, dim3(blocks_for(cells, 256)), dim3(256), 0, nullptr,
-                     n.dy.as<float>(), p, n.z3.as<float>(), rows, dz3);
-  // layer 3: dW3 = A2^T dZ3, db3, dA2 = dZ3 W3^T, dZ2 = dA2 SiLU'(z2)
-  hipLaunchKernelGGL(spo_dev::mlp_gemm_kernel, dim3(tiles * tiles), dim3(64), 0, nullptr, n.a2.as<float>(), 1L, H,
-                     dz3, H, 1L, static_cast<int>(rows), tiles, g + spo_dev::kMlpW3, H, 0,
-                     static_cast<const float*>(nullptr), static_cast<float*>(nullptr));
-  hipLaunchKernelGGL(spo_dev::mlp_column_sum_kernel, dim3(kMlpWidth), dim3(256), 0, nullptr, dz3, H,
-                     static_cast<const float*>(nullptr), rows, g + spo_dev::kMlpB3);
-  float* dz2 = n.d1.as<float>();
-  hipLaunchKernelGGL(spo_dev::mlp_gemm_kernel, dim3(static_cast<unsigned>(rows / 16 * tiles)), dim3(64), 0, nullptr,
-                     dz3, H, 1L, p + spo_dev::kMlpW3, 1L, H, kMlpWidth, tiles, dz2, H, 0,
-                     static_cast<const float*>(nullptr), static_cast<float*>(nullptr));
-  hipLaunchKernelGGL(spo_dev::mlp_silu_back_kernel, dim3(blocks_for(cells, 256)), dim3(256), 0, nullptr, dz2,
-                     n.z2.as<float>(), cells, dz2);
-  // layer 2
-  hipLaunchKernelGGL(spo_dev::mlp_gemm_kernel, dim3(tiles * tiles), dim3(64), 0, nullptr, n.a1.as<float>(), 1L, H,
-                     dz2, H, 1L, static_cast<int>(rows), tiles, g + spo_dev::kMlpW2, H, 0,
-                     static_cast<const float*>(nullptr), static_cast<float*>(nullptr));
-  hipLaunchKernelGGL(spo_dev::mlp_column_sum_kernel, dim3(kMlpWidth), dim3(256), 0, nullptr, dz2, H,
-                     static_cast<const float*>(nullptr), rows, g + spo_dev::kMlpB2);
-  float* dz1 = n.d2.as<float>();
-  hipLaunchKernelGGL(spo_dev::mlp_gemm_kernel, dim3(static_cast<unsigned>(rows / 16 * tiles)), dim3(64), 0, nullptr,
-                     dz2, H, 1L, p + spo_dev::kMlpW2, 1L, H, kMlpWidth, tiles, dz1, H, 0,
-                     static_cast<const float*>(nullptr), static_cast<float*>(nullptr));
-  hipLaunchKernelGGL(spo_dev::mlp_silu_back_kernel, dim3(blocks_for(cells, 256)), dim3(256), 0, nullptr, dz1,
-                     n.z1.as<float>(), cells, dz1);
-  // layer 1
-  hipLaunchKernelGGL(spo_dev::mlp_input_grad_kernel, dim3(spo_dev::kMlpIn * kMlpWidth), dim3(256), 0, nullptr, x, dz1,
-                     rows, g);
-  hipLaunchKernelGGL(spo_dev::mlp_column_sum_kernel, dim3(kMlpWidth), dim3(256), 0, nullptr, dz1, H,
-                     static_cast<const float*>(nullptr), rows, g + spo_dev::kMlpB1);
-  HIP_CHECK(hipGetLastError());
+void mlp_make_tape(spo_hip_mlp& n) {
+  if (n.tape.a1) return;
+  const std::size_t rows = n.batch, cells = rows * spo_dev::kMlpWidth;
+  n.operands = Buffer(4 * cells * sizeof(short));
+  n.values = Buffer(4 * cells * sizeof(float));
+  n.errors = Buffer(2 * rows * sizeof(float));
+  short* o = n.operands.as<short>();
+  float* f = n.values.as<float>();
+  float* e = n.errors.as<float>();
+  n.tape = {o, o + cells, o + 2 * cells, o + 3 * cells, f, f + cells, f + 2 * cells, f + 3 * cells, e, e + rows};
 }
 
-void mlp_adam(spo_hip_mlp& n, float lr) {
-  constexpr float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
-  ++n.adam_step;
-  const float c1 = 1.0f - std::pow(beta1, static_cast<float>(n.adam_step));
-  const float c2 = 1.0f - std::pow(beta2, static_cast<float>(n.adam_step));
-  hipLaunchKernelGGL(spo_dev::mlp_adam_kernel, dim3(blocks_for(spo_dev::kMlpParams, 256)), dim3(256), 0, nullptr,
-                     n.params.as<float>(), n.grad.as<float>(), n.m.as<float>(), n.v.as<float>(), spo_dev::kMlpParams,
-                     lr, beta1, beta2, eps, c1, c2);
+// One pass over the batch at x, t, then Adam, or the gradient to grad_out.
+void mlp_step(spo_hip_mlp& n, const float* x, const float* t, float* loss, float* grad_out, float lr) {
+  spo_dev::MlpAdam adam{n.params.as<float>(), n.m.as<float>(), n.v.as<float>(), grad_out, lr, 0.9f, 0.999f, 1e-8f,
+                        1.0f, 1.0f};
+  if (!grad_out) {
+    ++n.adam_step;
+    adam.c1 = 1.0f - std::pow(adam.beta1, static_cast<float>(n.adam_step));
+    adam.c2 = 1.0f - std::pow(adam.beta2, static_cast<float>(n.adam_step));
+  }
+  hipLaunchKernelGGL(spo_dev::mlp_pass_kernel, dim3(n.batch / spo_dev::kMlpRows), dim3(256), 0, nullptr, x, t,
+                     long(n.batch), n.params.as<float>(), n.frag.as<short>(), n.tape);
+  HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(spo_dev::mlp_update_kernel, dim3(spo_dev::kMlpUpdateBlocks), dim3(256), 0, nullptr, adam,
+                     n.frag.as<short>(), n.tape, x, long(n.batch), loss);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -1770,22 +1734,16 @@ int spo_hip_mlp_create(int batch, spo_hip_mlp** out) {
     require_device();
     auto n = std::make_unique<spo_hip_mlp>();
     n->batch = batch;
-    n->capacity = std::max<long>(batch, 1L << 16);
-    const std::size_t pb = spo_dev::kMlpParams * sizeof(float);
+    const std::size_t pb = spo_dev::kMlpParams * sizeof(float), fb = spo_dev::kMlpFragments * sizeof(short);
     n->params = Buffer(pb);
+    n->frag = Buffer(fb);
     n->grad = Buffer(pb);
     n->m = Buffer(pb);
     n->v = Buffer(pb);
     HIP_CHECK(hipMemset(n->params.as<void>(), 0, pb));
+    HIP_CHECK(hipMemset(n->frag.as<void>(), 0, fb));
     HIP_CHECK(hipMemset(n->m.as<void>(), 0, pb));
     HIP_CHECK(hipMemset(n->v.as<void>(), 0, pb));
-    const std::size_t rows = static_cast<std::size_t>(n->capacity);
-    n->x = Buffer(rows * spo_dev::kMlpIn * sizeof(float));
-    n->t = Buffer(rows * sizeof(float));
-    n->y = Buffer(rows * sizeof(float));
-    n->dy = Buffer(rows * sizeof(float));
-    for (Buffer* b : {&n->z1, &n->a1, &n->z2, &n->a2, &n->z3, &n->a3, &n->d1, &n->d2})
-      *b = Buffer(rows * kMlpWidth * sizeof(float));
     *out = n.release();
   });
 }
@@ -1803,6 +1761,9 @@ int spo_hip_mlp_set_params(spo_hip_mlp* mlp, const float* params) {
     HIP_CHECK(hipMemset(mlp->m.as<void>(), 0, pb));
     HIP_CHECK(hipMemset(mlp->v.as<void>(), 0, pb));
     mlp->adam_step = 0;
+    hipLaunchKernelGGL(spo_dev::mlp_fragment_kernel, dim3(blocks_for(2L * spo_dev::kMlpWidth * spo_dev::kMlpWidth, 256)),
+                       dim3(256), 0, nullptr, mlp->params.as<float>(), mlp->frag.as<short>());
+    HIP_CHECK(hipGetLastError());
   });
 }
 
@@ -1817,12 +1778,14 @@ int spo_hip_mlp_gradient(spo_hip_mlp* mlp, const float* x, const float* t, float
   return guarded([&] {
     if (!mlp || !x || !t || !loss || !grad) throw Status(SPO_HIP_E_ARGUMENT, "spo_hip_mlp_gradient: NULL argument");
     const long rows = mlp->batch;
-    HIP_CHECK(hipMemcpy(mlp->x.as<void>(), x, rows * spo_dev::kMlpIn * sizeof(float), hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemcpy(mlp->t.as<void>(), t, rows * sizeof(float), hipMemcpyHostToDevice));
-    Buffer l(sizeof(float));
-    mlp_forward(*mlp, rows, mlp->x.as<float>());
-    mlp_backward(*mlp, rows, mlp->x.as<float>(), mlp->t.as<float>(), l.as<float>());
-    HIP_CHECK(hipMemcpy(loss, l.as<void>(), sizeof(float), hipMemcpyDeviceToHost));
+    float* dx = at_least(mlp->x, mlp->x_values, rows * spo_dev::kMlpIn);
+    float* dt = at_least(mlp->t, mlp->t_values, rows);
+    float* dl = at_least(mlp->losses, mlp->loss_values, 1);
+    HIP_CHECK(hipMemcpy(dx, x, rows * spo_dev::kMlpIn * sizeof(float), hipMemcpyHostToDevice));
+    HIP_CHECK(hipMemcpy(dt, t, rows * sizeof(float), hipMemcpyHostToDevice));
+    mlp_make_tape(*mlp);
+    mlp_step(*mlp, dx, dt, dl, mlp->grad.as<float>(), 0.0f);
+    HIP_CHECK(hipMemcpy(loss, dl, sizeof(float), hipMemcpyDeviceToHost));
     HIP_CHECK(hipMemcpy(grad, mlp->grad.as<void>(), spo_dev::kMlpParams * sizeof(float), hipMemcpyDeviceToHost));
   });
 }
@@ -1832,33 +1795,38 @@ int spo_hip_mlp_train(spo_hip_mlp* mlp, long n, const float* x, const float* t, 
     if (!mlp || !x || !t || !losses) throw Status(SPO_HIP_E_ARGUMENT, "spo_hip_mlp_train: NULL argument");
     if (n < mlp->batch || n % mlp->batch != 0 || steps < 0)
       throw Status(SPO_HIP_E_ARGUMENT, "spo_hip_mlp_train: n must be a positive multiple of the batch");
-    Buffer dx = upload(x, std::size_t(n) * spo_dev::kMlpIn * sizeof(float));
-    Buffer dt = upload(t, std::size_t(n) * sizeof(float));
-    Buffer dl(std::size_t(std::max(steps, 1)) * sizeof(float));
-    const long rows = mlp->batch;
+    if (steps == 0) return;
+    // Only the rows that these steps reach.
+    const long rows = mlp->batch, used = std::min(n, steps * rows);
+    float* dx = at_least(mlp->x, mlp->x_values, used * spo_dev::kMlpIn);
+    float* dt = at_least(mlp->t, mlp->t_values, used);
+    float* dl = at_least(mlp->losses, mlp->loss_values, steps);
+    HIP_CHECK(hipMemcpy(dx, x, std::size_t(used) * spo_dev::kMlpIn * sizeof(float), hipMemcpyHostToDevice));
+    HIP_CHECK(hipMemcpy(dt, t, std::size_t(used) * sizeof(float), hipMemcpyHostToDevice));
+    mlp_make_tape(*mlp);
     for (int s = 0; s < steps; ++s) {
       const long off = (static_cast<long>(s) * rows) % n;
-      const float* xs = dx.as<float>() + off * spo_dev::kMlpIn;
-      mlp_forward(*mlp, rows, xs);
-      mlp_backward(*mlp, rows, xs, dt.as<float>() + off, dl.as<float>() + s);
-      mlp_adam(*mlp, lr);
+      mlp_step(*mlp, dx + off * spo_dev::kMlpIn, dt + off, dl + s, nullptr, lr);
     }
-    if (steps > 0) HIP_CHECK(hipMemcpy(losses, dl.as<void>(), steps * sizeof(float), hipMemcpyDeviceToHost));
+    HIP_CHECK(hipMemcpy(losses, dl, steps * sizeof(float), hipMemcpyDeviceToHost));
   });
 }
 
 int spo_hip_mlp_predict(spo_hip_mlp* mlp, long n, const float* x, float* y) {
   return guarded([&] {
     if (!mlp || (n > 0 && (!x || !y)) || n < 0) throw Status(SPO_HIP_E_ARGUMENT, "spo_hip_mlp_predict: bad arguments");
+    constexpr long kChunk = 1L << 20;  // rows per launch: 28 MB of device memory
     for (long done = 0; done < n;) {
-      const long chunk = std::min(mlp->capacity, n - done);
-      const long rows = (chunk + 15) / 16 * 16;  // the tail padded with zero rows
-      HIP_CHECK(hipMemset(mlp->x.as<void>(), 0, rows * spo_dev::kMlpIn * sizeof(float)));
-      HIP_CHECK(hipMemcpy(mlp->x.as<void>(), x + done * spo_dev::kMlpIn, chunk * spo_dev::kMlpIn * sizeof(float),
-                          hipMemcpyHostToDevice));
-      mlp_forward(*mlp, rows, mlp->x.as<float>());
-      HIP_CHECK(hipMemcpy(y + done, mlp->y.as<void>(), chunk * sizeof(float), hipMemcpyDeviceToHost));
-      done += chunk;
+      const long rows = std::min(kChunk, n - done);
+      float* dx = at_least(mlp->x, mlp->x_values, rows * spo_dev::kMlpIn);
+      float* dy = at_least(mlp->y, mlp->y_values, rows);
+      HIP_CHECK(hipMemcpy(dx, x + done * spo_dev::kMlpIn, rows * spo_dev::kMlpIn * sizeof(float), hipMemcpyHostToDevice));
+      const long tiles = (rows + spo_dev::kMlpRows - 1) / spo_dev::kMlpRows;
+      hipLaunchKernelGGL(spo_dev::mlp_predict_kernel, dim3(static_cast<unsigned>(std::min(tiles, 2048L))), dim3(256), 0,
+                         nullptr, dx, mlp->params.as<float>(), mlp->frag.as<short>(), rows, dy);
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipMemcpy(y + done, dy, rows * sizeof(float), hipMemcpyDeviceToHost));
+      done += rows;
     }
   });
 }

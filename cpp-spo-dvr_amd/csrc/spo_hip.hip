@@ -147,6 +147,24 @@ Buffer factor_lo(const double* p, std::size_t n, double factor = 1.0) {
   }
 }
 
+// The two entries (lane parity 0 and 1) of the sign-split rotation table for the factor x + i y.
+template <typename T>
+void set_rot_entries(spo_dev::RotEntry<T>* e, double x, double y) {
+  const cx<T> w = to_storage<T>(x, y);
+  e[0].x = w.x;
+  e[0].y = -w.y;
+  e[1].x = w.x;
+  e[1].y = w.y;
+  if constexpr (sizeof(T) == 4) {
+    const float lo_x = static_cast<float>(x - static_cast<double>(w.x));
+    const float lo_y = static_cast<float>(y - static_cast<double>(w.y));
+    e[0].lo_x = lo_x;
+    e[0].lo_y = -lo_y;
+    e[1].lo_x = lo_x;
+    e[1].lo_y = lo_y;
+  }
+}
+
 template <typename T>
 Buffer upload_real(const double* p, std::size_t n) {
   std::vector<T> v(p, p + n);
@@ -401,9 +419,13 @@ struct State final : spo_hip_backend {
   Buffer shift_f, shift_b, s2sc, legendre, block_first, block_size, block_offset, rot_block, rep_of, op_of, phi_index;
   Buffer exp_table, legendre_t;
   Buffer frag_fwd, frag_bwd, fwd_offset, bwd_offset, site_order, rot_pm, lo_fwd, lo_bwd, hi_fwd, hi_bwd;
+  // interaction_kernel_inplace (build_angular_plan): its tables, and the low parts' fragments of L (complex64)
+  Buffer ang_tasks, ang_free, ang_phi_map, ang_sites, ang_rot;
+  spo_dev::AngularPlan ang = {};
+  bool build_angular_plan(const spo_hip_tables* t, const std::vector<int>& offsets, int r1, int r2);
+  void run_interaction_inplace(const Variant& v);
   int max_jt = 1;
   int frag_fwd_count = 0, frag_bwd_count = 0;
-  bool v_buf = false;  // v_variants are interaction_buf_kernel instantiations
   int legendre_size = 0;
   std::size_t zr_lds = 0, xy_lds = 0, v_lds = 0;
   std::unique_ptr<DevicePlan<T>> plan_z, plan_r, plan_x, plan_y, plan_phi;
@@ -423,7 +445,7 @@ struct State final : spo_hip_backend {
   void run_zr(const Variant& v, bool half, cx<T>* row_out = nullptr, int row = -1);
   void run_xy(const Variant& v, bool half, bool kinetic_only, cx<T>* data = nullptr,
               const spo_dev::Shape* on = nullptr);
-  void run_interaction_mfma(const Variant& v);
+  void run_interaction(const Variant& v);
   void tune();
   void scattering_kinetic(bool half, bool kinetic_only);
 
@@ -507,11 +529,15 @@ void State<T>::run_xy(const Variant& v, bool half, bool kinetic_only, cx<T>* dat
 }
 
 template <typename T>
-void State<T>::run_interaction_mfma(const Variant& v) {
+void State<T>::run_interaction(const Variant& v) {
   cx<T>* ps = psi.as<cx<T>>();
   spo_dev::AngularTables at{legendre.as<double>(),  block_first.as<int>(), block_size.as<int>(),
                             block_offset.as<int>(), rot_block.as<int>(),   rep_of.as<int>(),
                             op_of.as<int>(),        phi_index.as<int>()};
+  if (v.kind == spo_dev::InteractionKind::in_place) {
+    run_interaction_inplace(v);
+    return;
+  }
   const int tiles = (s.n_zr_pot + 7) / 8;
   const int pair = s.n_xy % 8 == 0 ? 1 : 0;
   const cx<double>* sp = spec.as<cx<double>>();
@@ -526,7 +552,7 @@ void State<T>::run_interaction_mfma(const Variant& v) {
   const T* fb = frag_bwd.as<T>();
   int mj = max_jt;
   const int grid = pair ? 2 * ((tiles + 1) / 2) * s.n_xy : tiles * s.n_xy;
-  if (v_buf) {
+  if (v.kind == spo_dev::InteractionKind::buffer) {
     const cx<T>* rp = rot_pm.as<cx<T>>();
     const unsigned* lf = lo_fwd.as<unsigned>();
     const unsigned* lb = lo_bwd.as<unsigned>();
@@ -545,6 +571,146 @@ void State<T>::run_interaction_mfma(const Variant& v) {
                   const_cast<cx<T>**>(&rh), const_cast<cx<T>**>(&ssc), const_cast<T**>(&ep),
                   const_cast<cx<T>**>(&rl)};
   launch(v.fn, grid, v.threads, v.lds, stream, args);
+}
+
+template <typename T>
+void State<T>::run_interaction_inplace(const Variant& v) {
+  cx<T>* ps = psi.as<cx<T>>();
+  const cx<double>* sp = spec.as<cx<double>>();
+  spo_dev::AngularPlan plan = ang;
+  plan.rows = s.n_theta * v.columns;
+  plan.inv_rows = spo_dev::inverse_of(plan.rows);
+  const int tiles = (s.n_zr_pot + v.columns - 1) / v.columns;
+  const unsigned grid = 8u * plan.sites_per_xcd * 2u * ((tiles + 1) / 2);
+  const int* rep = rep_of.as<int>();
+  const int* op = op_of.as<int>();
+  const T* ff = frag_fwd.as<T>();
+  const T* fb = frag_bwd.as<T>();
+  const unsigned* lf = lo_fwd.as<unsigned>();
+  const unsigned* lb = lo_bwd.as<unsigned>();
+  const cx<T>* et = exp_table.as<cx<T>>();
+  const cx<T>* rp = ang_rot.as<cx<T>>();
+  const cx<T>* rh = rot_half.as<cx<T>>();
+  const cx<T>* ssc = s2sc.as<cx<T>>();
+  const cx<T>* tp = plan_phi->tw();
+  const T* ep = plan_phi->tw_eps();
+  void* args[] = {&ps, const_cast<cx<double>**>(&sp), &s, &plan, const_cast<int**>(&rep), const_cast<int**>(&op),
+                  const_cast<T**>(&ff), const_cast<T**>(&fb), const_cast<unsigned**>(&lf),
+                  const_cast<unsigned**>(&lb), const_cast<cx<T>**>(&et), const_cast<cx<T>**>(&rp),
+                  const_cast<cx<T>**>(&rh), const_cast<cx<T>**>(&ssc), const_cast<cx<T>**>(&tp),
+                  const_cast<T**>(&ep)};
+  launch(v.fn, grid, v.threads, v.lds, stream, args);
+}
+
+// The tables of interaction_kernel_inplace (the fragments themselves are frag_fwd and frag_bwd); false where the blocks
+// m and -m do not share their Legendre matrix up to the sign and their rotation factors, which the kernel relies on.
+template <typename T>
+bool State<T>::build_angular_plan(const spo_hip_tables* t, const std::vector<int>& offsets, int r1, int r2) {
+  const int mm = s.mj_max, n_tt = (s.n_theta + 15) / 16, k_bwd = (s.n_theta + 3) / 4;
+  std::vector<int> fo(s.n_blocks), bo(s.n_blocks);
+  int nf = 0, nb_count = 0, base = mm;
+  for (int b = 0; b < s.n_blocks; ++b) {
+    fo[b] = nf;
+    nf += n_tt * ((t->block_size[b] + 3) / 4);
+    bo[b] = nb_count;
+    nb_count += ((t->block_size[b] + 15) / 16) * k_bwd;
+    if (t->block_size[b] > t->block_size[base]) base = b;
+  }
+  // Rotation factors: one row per row of the longest block where every block's rows are a run of those (the rows of
+  // one J are the same for every mJ), else one per basis function.
+  auto same_row = [&](int i, int j) {
+    for (int ir = 0; ir < s.nr; ++ir)
+      for (int c = 0; c < 2; ++c)
+        if (t->rotation_half[2 * (i + std::size_t(s.n_rot) * ir) + c] !=
+            t->rotation_half[2 * (j + std::size_t(s.n_rot) * ir) + c])
+          return false;
+    return true;
+  };
+  std::vector<int> rot_first(s.n_blocks, -1);
+  const int bf = t->block_first[base], bn = t->block_size[base];
+  bool shared = true;
+  for (int b = 0; b < s.n_blocks && shared; ++b) {
+    for (int o = 0; o + t->block_size[b] <= bn && rot_first[b] < 0; ++o) {
+      bool all = true;
+      for (int j = 0; j < t->block_size[b] && all; ++j) all = same_row(t->block_first[b] + j, bf + o + j);
+      if (all) rot_first[b] = o;
+    }
+    shared = rot_first[b] >= 0;
+  }
+  const int rot_rows = shared ? bn : s.n_rot, rot_from = shared ? bf : 0;
+  if (!shared)
+    for (int b = 0; b < s.n_blocks; ++b) rot_first[b] = t->block_first[b];
+  std::vector<spo_dev::RotEntry<T>> pm(2 * std::size_t(rot_rows) * s.nr, spo_dev::RotEntry<T>{});
+  for (int row = 0; row < rot_rows; ++row)
+    for (int ir = 0; ir < s.nr; ++ir) {
+      const std::size_t from = 2 * (row + rot_from + std::size_t(s.n_rot) * ir);
+      set_rot_entries(pm.data() + spo_dev::rot_pm_index(row, ir, s.nr, 0), t->rotation_half[from],
+                      t->rotation_half[from + 1]);
+    }
+  std::vector<spo_dev::AngularTask> tasks;
+  std::vector<char> used(s.n_phi, 0);
+  const int cb = sizeof(cx<T>), fragment = 64 * sizeof(T);
+  for (int m = 0; m <= mm; ++m) {
+    const int b[2] = {mm + m, mm - m}, nb = t->block_size[b[0]];
+    bool plus = t->block_size[b[1]] == nb && rot_first[b[1]] == rot_first[b[0]], minus = plus;
+    for (int k = 0; k < s.n_theta * nb && (plus || minus); ++k) {
+      plus = plus && t->legendre[offsets[b[0]] + k] == t->legendre[offsets[b[1]] + k];
+      minus = minus && t->legendre[offsets[b[0]] + k] == -t->legendre[offsets[b[1]] + k];
+    }
+    if (!plus && !minus) return false;
+    spo_dev::AngularTask task{};
+    for (int side = 0; side < 2; ++side) {
+      const int place = spo_dev::phi_place(side && m ? s.n_phi - m : m, r1, r2), first = t->block_first[b[side]];
+      used[place] = 1;
+      task.psi[side] = first * s.n_zr * cb;
+      task.place[side] = place * cb;
+      if (s.ichn >= first && s.ichn < first + nb && !(side && m == 0)) {
+        ang.task_initial = m;
+        ang.side_initial = side;
+        ang.j_initial = s.ichn - first;
+      }
+    }
+    task.nb = nb;
+    task.fwd = fo[b[0]] * fragment;
+    task.bwd = bo[b[0]] * fragment;
+    task.negate = plus ? 0 : 1;
+    task.rot = rot_first[b[0]] * s.nr * 32;
+    tasks.push_back(task);
+  }
+  std::vector<int> free_places;
+  for (int p = 0; p < s.n_phi; ++p)
+    if (!used[p]) free_places.push_back(p);
+  ang.n_free = static_cast<int>(free_places.size());
+  free_places.push_back(0);  // never empty
+  std::vector<int> map;
+  for (int op = 0; op < shape.n_operations; ++op)
+    for (int p = 0; p < s.n_phi; ++p) map.push_back(t->phi_index[spo_dev::phi_frequency(p, r1, r2) + s.n_phi * op]);
+  // Sites sorted by representative, an eighth to each XCD (rounded up; the rest of the positions hold none).
+  std::vector<int> sorted(s.n_xy);
+  for (int i = 0; i < s.n_xy; ++i) sorted[i] = i;
+  std::stable_sort(sorted.begin(), sorted.end(),
+                   [&](int x, int y) { return t->representative_of[x] < t->representative_of[y]; });
+  const int per = (s.n_xy + 7) / 8;
+  std::vector<int> sites(8 * std::size_t(per), -1);
+  for (int x = 0; x < 8; ++x)
+    for (int k = 0; k < per; ++k)
+      if (per * x + k < s.n_xy) sites[8 * k + x] = sorted[per * x + k];
+  ang_tasks = upload(tasks.data(), tasks.size() * sizeof(spo_dev::AngularTask));
+  ang_free = upload(free_places.data(), free_places.size() * sizeof(int));
+  ang_phi_map = upload(map.data(), map.size() * sizeof(int));
+  ang_sites = upload(sites.data(), sites.size() * sizeof(int));
+  ang_rot = upload(pm.data(), pm.size() * sizeof(spo_dev::RotEntry<T>));
+  ang.tasks = ang_tasks.as<spo_dev::AngularTask>();
+  ang.n_tasks = static_cast<int>(tasks.size());
+  ang.free_places = ang_free.as<int>();
+  ang.phi_map = ang_phi_map.as<int>();
+  ang.site_order = ang_sites.as<int>();
+  ang.sites_per_xcd = per;
+  ang.inv_nr = spo_dev::inverse_of(s.nr);
+  ang.rot_rows = rot_rows;
+  ang.frag_fwd = nf;
+  ang.frag_bwd = nb_count;
+  return true;
 }
 
 // The launch tuner. The variants of one family differ only in block sizes and tiles; the compiler may contract
@@ -627,7 +793,7 @@ void State<T>::tune() {
   // The scattering wave is zero here, and every kernel maps zero to zero.
   zr_pick = pick(zr_variants, "zr", true, [&](const Variant& v) { run_zr(v, false); });
   xy_pick = pick(xy_variants, "xy", false, [&](const Variant& v) { run_xy(v, false, false); });
-  v_pick = pick(v_variants, "interaction", false, [&](const Variant& v) { run_interaction_mfma(v); });
+  v_pick = pick(v_variants, "interaction", false, [&](const Variant& v) { run_interaction(v); });
   HIP_CHECK(hipStreamSynchronize(stream));
 }
 
@@ -696,11 +862,12 @@ void State<T>::step_block(bool specular_half, int scattering, bool kinetic_only)
   const cx<T>* rh = rot_half.as<cx<T>>();
   const cx<T>* ssc = s2sc.as<cx<T>>();
   if (!v_variants.empty()) {
-    timed("specular_coupling", [&] {
-      hipLaunchKernelGGL(spo_dev::specular_coupling_kernel<T>, dim3(blocks_for(long(s.n_zr_pot) * s.n_xy, 256)),
-                         dim3(256), 0, stream, ps, sp, s, rh, ssc);
-    });
-    timed("interaction", [&] { run_interaction_mfma(v_variants[v_pick]); });
+    if (v_variants[v_pick].kind != spo_dev::InteractionKind::in_place)
+      timed("specular_coupling", [&] {
+        hipLaunchKernelGGL(spo_dev::specular_coupling_kernel<T>, dim3(blocks_for(long(s.n_zr_pot) * s.n_xy, 256)),
+                           dim3(256), 0, stream, ps, sp, s, rh, ssc);
+      });
+    timed("interaction", [&] { run_interaction(v_variants[v_pick]); });
   } else if (v_fn) {
     const cx<T>* tp = plan_phi->tw();
     const T* lt = legendre_t.as<T>();
@@ -1037,7 +1204,7 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
   // run-time engine on the plane, else lines.
   if (spo_dev::zr_plane_lds<T>(s.nz, s.nr) <= lds_limit) b->zr_variants = spo_dev::zr_variants<T>(s.nz, s.nr);
   if (!b->zr_variants.empty()) {
-    for (const Variant& v : b->zr_variants) set_lds(v.fn, v.lds);
+    for (const Variant& v : b->zr_variants) set_lds(v.fn, lds_limit);  // one kernel serves planes of many sizes
     b->order_zr_factors(zr_full_values, zr_half_values, b->zr_variants[0].zr);
   } else if (std::size_t(s.n_zr) * cT <= lds_limit) {
     b->zr_fused = true;
@@ -1067,11 +1234,13 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
   b->v_lds = v_bytes(p2);
   if (b->v_lds > lds_limit) throw Status(SPO_HIP_E_NOT_SUPPORTED, "an angular column does not fit in LDS");
   set_lds(b->v_fn ? b->v_fn : reinterpret_cast<const void*>(spo_dev::interaction_kernel<T>), b->v_lds);
-  // Interaction with the theta contractions on MFMA: Legendre fragments in lane order, XCD-grouped site order.
-  // SPO_HIP_INTERACTION selects a variant for comparisons: "buf" (the buffer-addressed MFMA kernel where its shape
-  // conditions hold, else "mfma"; the complex64 default), "mfma" (MFMA contractions, fused register phi step; the
-  // FP64 default: 4.33 against 4.89 ms per launch at the DZ workload on MI355X), "mfma_staged" (MFMA contractions,
-  // staged LDS phi FFTs), "lds" (contractions on the vector units).
+  // Interaction with the theta contractions on MFMA: Legendre fragments in lane order, XCD-grouped site order. The
+  // default is interaction_kernel_inplace where its conditions hold (an instantiated phi length, at most 16 theta
+  // points and 16 J per block, 32-bit offsets within a site, one Legendre matrix for m and -m), followed in the list by
+  // the kernels below for the launch tuner.
+  // SPO_HIP_INTERACTION selects one of the others for comparisons: "buf" (the buffer-addressed MFMA kernel where its
+  // shape conditions hold, else "mfma"), "mfma" (MFMA contractions, fused register phi step), "mfma_staged" (MFMA
+  // contractions, staged LDS phi FFTs), "lds" (contractions on the vector units).
   {
     const char* env = std::getenv("SPO_HIP_INTERACTION");
     const std::string choice = env ? env : (sizeof(T) == 8 ? "mfma" : "buf");
@@ -1090,7 +1259,13 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
     // phi lengths with a buffer-kernel instantiation only (the reduced-JMax batch members' 28 and 40 points)
     const bool buf_candidate =
         choice == "buf" && !spo_dev::interaction_buf_variants<T>(s.n_phi, s.n_theta, s.n_blocks, bf16x3).empty();
-    if ((!variants.empty() || buf_candidate) && choice != "lds") {
+    int longest_block = 0;
+    for (int blk = 0; blk < s.n_blocks; ++blk) longest_block = std::max(longest_block, t->block_size[blk]);
+    std::vector<Variant> in_place;
+    if (!env && !bf16x3 && longest_block <= 16 && std::size_t(s.n_zr) * s.n_rot * cT < (std::size_t(1) << 31))
+      for (const Variant& v : spo_dev::interaction_inplace_variants<T>(s.n_phi, s.n_theta, long(s.n_zr_pot) * s.n_xy))
+        if (v.lds <= lds_limit) in_place.push_back(v);
+    if ((!variants.empty() || buf_candidate || !in_place.empty()) && choice != "lds") {
       const int n_tt = (s.n_theta + 15) / 16, k_bwd = (s.n_theta + 3) / 4;
       std::vector<int> fo(s.n_blocks), bo(s.n_blocks);
       int nf = 0, nbw = 0, max_nb = 0;
@@ -1139,6 +1314,47 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
       b->max_jt = (max_nb + 15) / 16;
       b->frag_fwd_count = nf;
       b->frag_bwd_count = nbw;
+      auto low_fragments = [&] {
+        if (sizeof(T) != 4 || b->lo_fwd.template as<void>()) return;
+        // bf16 fragments of a function of L, lane (i, q) element t = contraction row 4 t + q
+        // (legendre_low_product): forward A = L (theta = i, J = row), backward A = L^T (J = i, theta = row).
+        auto bf16 = [](double x) -> std::uint16_t {
+          const float f = static_cast<float>(x);
+          std::uint32_t u;
+          std::memcpy(&u, &f, 4);
+          u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even (the values are finite and small)
+          return static_cast<std::uint16_t>(u >> 16);
+        };
+        auto bf16_value = [&](double x) {
+          const std::uint32_t u = std::uint32_t(bf16(x)) << 16;
+          float f;
+          std::memcpy(&f, &u, 4);
+          return static_cast<double>(f);
+        };
+        auto fragments = [&](auto&& piece, Buffer& fwd, Buffer& bwd) {
+          std::vector<std::uint16_t> lf(256 * std::size_t(s.n_blocks), 0), lb(256 * std::size_t(s.n_blocks), 0);
+          for (int blk = 0; blk < s.n_blocks; ++blk) {
+            const int nb = t->block_size[blk];
+            const double* L = t->legendre + offsets[blk];  // (theta, J)
+            for (int lane = 0; lane < 64; ++lane)
+              for (int e = 0; e < 4; ++e) {
+                const int i = lane % 16, q = lane / 16, row = 4 * e + q;
+                if (i < s.n_theta && row < nb) lf[256 * std::size_t(blk) + 4 * lane + e] = bf16(piece(L[i * nb + row]));
+                if (row < s.n_theta && i < nb) lb[256 * std::size_t(blk) + 4 * lane + e] = bf16(piece(L[row * nb + i]));
+              }
+          }
+          fwd = upload(lf.data(), lf.size() * sizeof(std::uint16_t));
+          bwd = upload(lb.data(), lb.size() * sizeof(std::uint16_t));
+        };
+        if (bf16x3) {
+          // split-BF16x3: A_hi = bf16(L), A_lo = bf16(L - A_hi)
+          fragments([&](double l) { return l; }, b->hi_fwd, b->hi_bwd);
+          fragments([&](double l) { return l - bf16_value(l); }, b->lo_fwd, b->lo_bwd);
+        } else {
+          // the low part L - float(L) of the FP32 contraction
+          fragments([](double l) { return l - static_cast<double>(static_cast<float>(l)); }, b->lo_fwd, b->lo_bwd);
+        }
+      };
       // The buffer-addressed kernel where its shape conditions hold: one theta tile, blocks of at most 16 J, a
       // site column addressable with 32-bit offsets.
       if (choice == "buf" && s.n_theta <= 16 && max_nb <= 16 &&
@@ -1156,70 +1372,21 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
             for (int ir = 0; ir < s.nr; ++ir) {
               const double x = t->rotation_half[2 * (irot + std::size_t(s.n_rot) * ir)];
               const double y = t->rotation_half[2 * (irot + std::size_t(s.n_rot) * ir) + 1];
-              const cx<T> w = to_storage<T>(x, y);
-              const std::size_t e0 = spo_dev::rot_pm_index(irot, ir, s.nr, 0);
-              pm[e0].x = w.x;
-              pm[e0].y = -w.y;
-              pm[e0 + 1].x = w.x;
-              pm[e0 + 1].y = w.y;
-              if constexpr (sizeof(T) == 4) {
-                const float lo_x = static_cast<float>(x - static_cast<double>(w.x));
-                const float lo_y = static_cast<float>(y - static_cast<double>(w.y));
-                pm[e0].lo_x = lo_x;
-                pm[e0].lo_y = -lo_y;
-                pm[e0 + 1].lo_x = lo_x;
-                pm[e0 + 1].lo_y = lo_y;
-              }
+              set_rot_entries(pm.data() + spo_dev::rot_pm_index(irot, ir, s.nr, 0), x, y);
             }
           b->rot_pm = upload(pm.data(), pm.size() * sizeof(spo_dev::RotEntry<T>));
-          if (sizeof(T) == 4) {
-            // bf16 fragments of a function of L, lane (i, q) element t = contraction row 4 t + q
-            // (legendre_low_product): forward A = L (theta = i, J = row), backward A = L^T (J = i, theta = row).
-            auto bf16 = [](double x) -> std::uint16_t {
-              const float f = static_cast<float>(x);
-              std::uint32_t u;
-              std::memcpy(&u, &f, 4);
-              u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even (the values are finite and small)
-              return static_cast<std::uint16_t>(u >> 16);
-            };
-            auto bf16_value = [&](double x) {
-              const std::uint32_t u = std::uint32_t(bf16(x)) << 16;
-              float f;
-              std::memcpy(&f, &u, 4);
-              return static_cast<double>(f);
-            };
-            auto fragments = [&](auto&& piece, Buffer& fwd, Buffer& bwd) {
-              std::vector<std::uint16_t> lf(256 * std::size_t(s.n_blocks), 0), lb(256 * std::size_t(s.n_blocks), 0);
-              for (int blk = 0; blk < s.n_blocks; ++blk) {
-                const int nb = t->block_size[blk];
-                const double* L = t->legendre + offsets[blk];  // (theta, J)
-                for (int lane = 0; lane < 64; ++lane)
-                  for (int e = 0; e < 4; ++e) {
-                    const int i = lane % 16, q = lane / 16, row = 4 * e + q;
-                    if (i < s.n_theta && row < nb) lf[256 * std::size_t(blk) + 4 * lane + e] = bf16(piece(L[i * nb + row]));
-                    if (row < s.n_theta && i < nb) lb[256 * std::size_t(blk) + 4 * lane + e] = bf16(piece(L[row * nb + i]));
-                  }
-              }
-              fwd = upload(lf.data(), lf.size() * sizeof(std::uint16_t));
-              bwd = upload(lb.data(), lb.size() * sizeof(std::uint16_t));
-            };
-            if (bf16x3) {
-              // split-BF16x3: A_hi = bf16(L), A_lo = bf16(L - A_hi)
-              fragments([&](double l) { return l; }, b->hi_fwd, b->hi_bwd);
-              fragments([&](double l) { return l - bf16_value(l); }, b->lo_fwd, b->lo_bwd);
-            } else {
-              // the low part L - float(L) of the FP32 contraction
-              fragments([](double l) { return l - static_cast<double>(static_cast<float>(l)); }, b->lo_fwd, b->lo_bwd);
-            }
-          }
+          low_fragments();
           variants = buf;
-          b->v_buf = true;
         }
+      }
+      if (!in_place.empty() && b->build_angular_plan(t, offsets, in_place[0].r1, in_place[0].r2)) {
+        low_fragments();
+        variants.insert(variants.begin(), in_place.begin(), in_place.end());
       }
       if (!variants.empty()) {  // else the kernels chosen above (v_fn or the run-time-shaped one) stay
         b->v_variants = variants;
         b->v_c = 8;
-        for (const Variant& v : variants) set_lds(v.fn, v.lds);
+        for (const Variant& v : variants) set_lds(v.fn, lds_limit);
       }
     }
   }

@@ -33,7 +33,7 @@ std::vector<Variant> interaction_mfma_variants(int nphi, int n_theta, bool fused
   if (nphi == A && (fused || W == 8))                                                                        \
     out.push_back({fused ? reinterpret_cast<const void*>(spo_dev::interaction_mfma_kernel<T, A, NT, W, R1, R2>) \
                          : reinterpret_cast<const void*>(spo_dev::interaction_mfma_kernel<T, A, NT, W>),     \
-                   64 * W, W, lds});
+                   64 * W, W, lds, {}, InteractionKind::mfma});
   SPO_MFMA_SHAPES(X)
 #undef X
   return out;
@@ -49,13 +49,13 @@ std::vector<Variant> interaction_buf_variants(int nphi, int n_theta, int n_block
     if constexpr (sizeof(T) == 4) {
       if (nphi == 48 && n_blocks <= 64)
         out.push_back({reinterpret_cast<const void*>(spo_dev::interaction_buf_kernel<T, 48, 8, 12, 4, true>), 512,
-                       8, lds});
+                       8, lds, {}, InteractionKind::buffer});
     }
     return out;
   }
 #define X(A, W, R1, R2)                                                                                         \
   if (nphi == A && n_blocks <= 8 * W)                                                                           \
-    out.push_back({reinterpret_cast<const void*>(spo_dev::interaction_buf_kernel<T, A, W, R1, R2>), 64 * W, W, lds});
+    out.push_back({reinterpret_cast<const void*>(spo_dev::interaction_buf_kernel<T, A, W, R1, R2>), 64 * W, W, lds, {}, InteractionKind::buffer});
   SPO_BUF_SHAPES(X)
 #undef X
   return out;

@@ -63,3 +63,16 @@ def test_zr_plane_shapes(nz, nr):
 @pytest.mark.parametrize("nz,nr", [(22, 10), (28, 12)])
 def test_xy_line_lengths(nxy, nz, nr):
     _check(f"xy_{nxy}_{nz}_{nr}", _grid(nz, nr, nxy, 2), 200 + nxy + nz, blocks=((False, False), (True, True)))
+
+
+# Angular bases for every phi length with a kernel of its own (JMax, MJMax, two equal atoms), the longest block that it
+# takes (16 J), one J more (another kernel), and truncated mJ.
+@pytest.mark.parametrize("jmax,mjmax,homonuclear", [
+    (0, 0, True), (1, 1, False), (2, 2, True), (3, 3, False), (4, 4, True), (5, 5, False), (6, 6, True), (7, 7, False),
+    (8, 8, True), (9, 9, False), (10, 10, True), (11, 11, False), (12, 12, True), (14, 14, True), (15, 15, False),
+    (16, 16, True), (16, 16, False), (18, 18, True), (20, 20, True), (22, 20, True), (22, 22, True), (24, 23, True),
+    (24, 24, True), (28, 28, True), (30, 30, True), (12, 3, False), (24, 2, True)])
+@pytest.mark.parametrize("sym", [False, True])
+def test_angular_bases(jmax, mjmax, homonuclear, sym):
+    _check(f"ang_{jmax}_{mjmax}_{homonuclear}_{sym}",
+           _grid(22, 10, 4, jmax, mjmax=mjmax, HomoNuc=homonuclear, UseSymmetry=sym), 300 + 2 * jmax + mjmax)

@@ -240,11 +240,19 @@ __device__ __forceinline__ void rdft(cx<T>* v, int sign) {
     rdft_composite<5, 3, T>(v, sign);
   } else if constexpr (R == 16) {
     rdft_composite<4, 4, T>(v, sign);
+  } else if constexpr (R == 18) {
+    rdft_composite<9, 2, T>(v, sign);
+  } else if constexpr (R == 20) {
+    rdft_composite<5, 4, T>(v, sign);
+  } else if constexpr (R == 22) {
+    rdft_composite<11, 2, T>(v, sign);
   }
 }
 
-// The lengths rdft transforms.
-constexpr bool register_radix(int r) { return r >= 1 && r <= 16 && r != 13; }
+// The lengths rdft transforms (those above 16 only where a thread has 256 registers).
+constexpr bool register_radix(int r, int most = 16) {
+  return r >= 1 && r <= most && ((r <= 16 && r != 13) || r == 18 || r == 20 || r == 22);
+}
 
 // ---- one stage, whole sequences per round ---------------------------------------------------------------------
 // Sequence s starts at (s % INNER) * IS + (s / INNER) * OS (INNER = 0: at s * IS); elements ES apart.

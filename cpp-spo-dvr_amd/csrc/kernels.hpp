@@ -312,12 +312,15 @@ __global__ __launch_bounds__(64 * kProjectionWaves) void projection_kernel(cx<T>
 
 // ---------------------------------------------------------------------------------------------------------------
 // Analysis. One workgroup per (v, irotana): overlap over r with phi_vj(r) dR and the momentum shift, (x, y) FFT
-// (sign -, scale 1), pick the analysed diffraction slots (src/analysis/balint_kurti.cpp:52-72).
+// (sign -, scale 1), pick the analysed diffraction slots (src/analysis/balint_kurti.cpp:52-72). Every coefficient is
+// written. spec not NULL: the initial state's are taken from the specular wave at the fixed analysis surface instead
+// (:74-82), by the workgroup whose coefficient it is; phi_in(ir, v) the initial state's radial functions.
 template <typename T>
 __global__ void bk_scattering_kernel(const cx<T>* psi, Shape s, int iz_ana, int n_rot_ana, int n_dif,
                                      int n_states, const int* rot_index, const int* slots, const double* weights,
                                      const cx<double>* shift_f, double xy_scale, FftPlan plan_x, FftPlan plan_y,
-                                     cx<double>* bk) {
+                                     cx<double>* bk, const cx<double>* spec, int iz_sp, int initial,
+                                     const double* phi_in, double dr) {
   extern __shared__ unsigned char smem_raw[];
   cx<double>* ov = reinterpret_cast<cx<double>*>(smem_raw);
   const int task = blockIdx.x;
@@ -338,18 +341,16 @@ __global__ void bk_scattering_kernel(const cx<T>* psi, Shape s, int iz_ana, int 
   const SeqLayout xs{s.ny, s.ny, 1, 0, s.ny};
   lds_fft<double>(ov, ys, plan_y, -1);
   lds_fft<double>(ov, xs, plan_x, -1);
-  for (int idif = threadIdx.x; idif < n_dif; idif += blockDim.x)
-    bk[irotana * n_dif + idif + (long)n_states * v] = scale(ov[slots[idif]], xy_scale);
-}
-
-// The initial state from the specular wave at the fixed analysis surface (src/analysis/balint_kurti.cpp:74-82).
-__global__ inline void bk_specular_kernel(const cx<double>* spec, int nr, int iz_sp, int n_v, int n_states, int initial,
-                                   const double* phi_in, double dr, cx<double>* bk) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n_v) return;
-  cx<double> acc = {0.0, 0.0};
-  for (int ir = 0; ir < nr; ++ir) acc = acc + scale(spec[ir + nr * iz_sp], phi_in[ir + nr * v]);
-  bk[initial + (long)n_states * v] = scale(acc, dr);
+  for (int idif = threadIdx.x; idif < n_dif; idif += blockDim.x) {
+    const int is = irotana * n_dif + idif;
+    cx<double> c = scale(ov[slots[idif]], xy_scale);
+    if (spec && is == initial) {
+      cx<double> acc = {0.0, 0.0};
+      for (int ir = 0; ir < s.nr; ++ir) acc = acc + scale(spec[ir + s.nr * iz_sp], phi_in[ir + s.nr * v]);
+      c = scale(acc, dr);
+    }
+    bk[is + (long)n_states * v] = c;
+  }
 }
 
 // sums(k, ien) += c(k) exp(i E_ien t) dtAna, FP64 (src/analysis/s_matrix.cpp:49-56).
@@ -366,25 +367,6 @@ __global__ inline void s_accumulate_kernel(cx<double>* sums, const cx<double>* b
 
 // ---------------------------------------------------------------------------------------------------------------
 // Wave-packet utilities.
-__global__ inline void zero_kernel(cx<double>* p, long n) {
-  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) p[k] = cx<double>{0.0, 0.0};
-}
-
-template <typename T>
-__global__ void densities_kernel(const cx<T>* psi, Shape s, double* out) {
-  const int izr = blockIdx.x * blockDim.x + threadIdx.x;
-  if (izr >= s.n_zr) return;
-  double acc = 0.0;
-  for (int ixy = 0; ixy < s.n_xy; ++ixy)
-    for (int irot = 0; irot < s.n_rot; ++irot) {
-      const cx<T> v = psi[izr + (long)s.n_zr * (irot + (long)s.n_rot * ixy)];
-      const double a = hypot(double(v.x), double(v.y));
-      acc = acc + a * a;
-    }
-  out[izr] = acc;
-}
-
 // out (irot, ixy, ir) of Z index iz.
 template <typename T>
 __global__ void z_plane_kernel(const cx<T>* psi, Shape s, int iz, cx<double>* out) {

@@ -42,9 +42,14 @@ __device__ __forceinline__ int fast_div(int x, int n, unsigned inv) {
   return n == 1 ? x : static_cast<int>(__umulhi(static_cast<unsigned>(x), inv));
 }
 
-// Calls f with the radix as a compile-time constant.
-template <class F>
+// Calls f with the radix (at most MOST) as a compile-time constant.
+template <int MOST, class F>
 __device__ __forceinline__ void with_radix(int r, F&& f) {
+  if constexpr (MOST > 16) {
+    if (r == 18) return f(std::integral_constant<int, 18>{});
+    if (r == 20) return f(std::integral_constant<int, 20>{});
+    if (r == 22) return f(std::integral_constant<int, 22>{});
+  }
   switch (r) {
     case 1: f(std::integral_constant<int, 1>{}); break;
     case 2: f(std::integral_constant<int, 2>{}); break;
@@ -64,13 +69,15 @@ __device__ __forceinline__ void with_radix(int r, F&& f) {
     default: break;
   }
 }
-template <int R, class F>
+template <int MOST, int R, class F>
 __device__ __forceinline__ void with_radix(std::integral_constant<int, R>, F&& f) {
   f(std::integral_constant<int, R>{});
 }
 
 // The plane's shape as run-time values or as compile-time constants.
+template <int MOST>
 struct ZrRunTime {
+  static constexpr int kMost = MOST;  // the largest radix
   ZrShape s;
   __device__ __forceinline__ explicit ZrRunTime(const ZrShape& shape) : s(shape) {}
   __device__ __forceinline__ int nz() const { return s.nz; }
@@ -85,6 +92,7 @@ struct ZrRunTime {
 };
 template <int NZ, int NR, int A1, int A2, int B1, int B2>
 struct ZrStatic {
+  static constexpr int kMost = 16;
   static_assert(A1 * A2 == NR && B1 * B2 == NZ, "ZrStatic: radices must multiply to the lengths");
   __device__ __forceinline__ explicit ZrStatic(const ZrShape&) {}
   template <int V>
@@ -108,16 +116,15 @@ inline std::size_t zr_plane_lds(int nz, int nr) {
          (zr_twiddles_in_lds<T>() ? std::size_t(nz + nr) * 2 * sizeof(cx<T>) : 0);
 }
 
+// One plane through the passes: read from `plane`, every value of the result handed to out(iz, ir, value).
 // factor and factor_lo (complex64: its FP32 remainders, mul_hilo) in the order of zr_factor_order; eps_z, eps_r: the
 // complex64 twiddle tables' modulus corrections (twiddle()). FP64 keeps the twiddles in the cache, where they do not
 // compete with the plane for LDS bandwidth; complex64 holds them and their remainders in LDS.
-// row >= 0: psi is only read, and Z row `row` of each transformed plane (NR values) goes to row_out[plane * NR + ir]
-// (the inverse r passes run for that row alone); row < 0: psi is transformed in place and row_out is unused.
-template <typename T, class Dims, int THREADS>
-__global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape shape, const cx<T>* table_z,
-                                                             const cx<T>* table_r, const cx<T>* factor, const T* eps_z,
-                                                             const T* eps_r, const cx<T>* factor_lo, cx<T>* row_out,
-                                                             int row) {
+// row >= 0: only Z row `row` of the result is formed (the inverse r passes run for that row alone).
+template <typename T, class Dims, int THREADS, class Out>
+__device__ __forceinline__ void zr_transform(const cx<T>* plane, const ZrShape& shape, const cx<T>* table_z,
+                                             const cx<T>* table_r, const cx<T>* factor, const T* eps_z, const T* eps_r,
+                                             const cx<T>* factor_lo, int row, Out&& out) {
   extern __shared__ unsigned char smem_raw[];
   cx<T>* t = reinterpret_cast<cx<T>*>(smem_raw);
   const Dims d(shape);
@@ -128,7 +135,6 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
   const auto b1 = d.b1();
   const auto b2 = d.b2();
   const int ld = zr_row(nr);
-  cx<T>* plane = psi + static_cast<long>(blockIdx.x) * (nz * nr);
   const int tid = threadIdx.x;
   const cx<T>* lo_r = nullptr;
   const cx<T>* lo_z = nullptr;
@@ -156,7 +162,7 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
   }
 
   // r forward, radix a1: butterfly (iz, j < a2) from HBM.
-  with_radix(a1, [&](auto radix) {
+  with_radix<Dims::kMost>(a1, [&](auto radix) {
     constexpr int R = decltype(radix)::value;
     const int n = nz * a2;
 #pragma unroll 2
@@ -174,7 +180,7 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
   });
   __syncthreads();
   // r forward, radix a2: butterfly (iz, k1 < a1), lanes along iz.
-  with_radix(a2, [&](auto radix) {
+  with_radix<Dims::kMost>(a2, [&](auto radix) {
     constexpr int R = decltype(radix)::value;
     if constexpr (R > 1) {
       const int n = nz * a1;
@@ -193,7 +199,7 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
   });
   __syncthreads();
   // Z forward, radix b1: butterfly (place in the row, j < b2), lanes along the row.
-  with_radix(b1, [&](auto radix) {
+  with_radix<Dims::kMost>(b1, [&](auto radix) {
     constexpr int R = decltype(radix)::value;
     const int n = nr * b2, step = b2 * ld;
     for (int b = tid; b < n; b += THREADS) {
@@ -209,7 +215,7 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
   });
   __syncthreads();
   // Z forward radix b2, x factor, Z inverse radix b2: butterfly (place in the row, k1 < b1).
-  with_radix(b2, [&](auto radix) {
+  with_radix<Dims::kMost>(b2, [&](auto radix) {
     constexpr int R = decltype(radix)::value;
     const int n = nr * b1;
     for (int b = tid; b < n; b += THREADS) {
@@ -231,7 +237,7 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
   });
   __syncthreads();
   // Z inverse, radix b1.
-  with_radix(b1, [&](auto radix) {
+  with_radix<Dims::kMost>(b1, [&](auto radix) {
     constexpr int R = decltype(radix)::value;
     const int n = nr * b2, step = b2 * ld;
     for (int b = tid; b < n; b += THREADS) {
@@ -247,7 +253,7 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
   });
   __syncthreads();
   // r inverse, radix a2 (row mode: of that row alone).
-  with_radix(a2, [&](auto radix) {
+  with_radix<Dims::kMost>(a2, [&](auto radix) {
     constexpr int R = decltype(radix)::value;
     if constexpr (R > 1) {
       const int n = nz * a1;
@@ -267,7 +273,7 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
   });
   __syncthreads();
   // r inverse, radix a1, to HBM.
-  with_radix(a1, [&](auto radix) {
+  with_radix<Dims::kMost>(a1, [&](auto radix) {
     constexpr int R = decltype(radix)::value;
     const int n = nz * a2;
     for (int b = tid; b < n; b += THREADS) {
@@ -278,11 +284,53 @@ __global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape
 #pragma unroll
       for (int r = 0; r < R; ++r) v[r] = src[r * a2];
       rdft<R, T>(v, +1);
-      cx<T>* out = row >= 0 ? row_out + static_cast<long>(blockIdx.x) * nr + j : plane + (iz * nr + j);
 #pragma unroll
-      for (int r = 0; r < R; ++r) out[r * a2] = v[r];
+      for (int r = 0; r < R; ++r) out(iz, j + r * a2, v[r]);
     }
   });
+}
+
+// T_Zr of one (irot, ixy) plane per workgroup. row >= 0: psi is only read, and Z row `row` of each transformed plane
+// (NR values) goes to row_out[plane * NR + ir]; row < 0: psi is transformed in place and row_out is unused.
+template <typename T, class Dims, int THREADS>
+__global__ __launch_bounds__(THREADS) void zr_inplace_kernel(cx<T>* psi, ZrShape shape, const cx<T>* table_z,
+                                                             const cx<T>* table_r, const cx<T>* factor, const T* eps_z,
+                                                             const T* eps_r, const cx<T>* factor_lo, cx<T>* row_out,
+                                                             int row) {
+  const Dims d(shape);
+  const auto nr = d.nr();
+  cx<T>* plane = psi + static_cast<long>(blockIdx.x) * (d.nz() * nr);
+  cx<T>* line = row_out + static_cast<long>(blockIdx.x) * nr;
+  zr_transform<T, Dims, THREADS>(plane, shape, table_z, table_r, factor, eps_z, eps_r, factor_lo, row,
+                                 [&](int iz, int ir, cx<T> v) {
+                                   if (row >= 0)
+                                     line[ir] = v;
+                                   else
+                                     plane[iz * nr + ir] = v;
+                                 });
+}
+
+// The specular grid's whole step by one workgroup, for a grid that fits in LDS: its kinetic step, then (potential != 0)
+// exp(-i vasy dt) between rot(dt/2) for iz >= nzpot and the Z and r absorbers
+// (src/propagation/specular_operator.cpp:40-71). The grid is a few thousand points and the step is a chain of passes:
+// one workgroup does it in 11 us at 128 x 16 and 32 us at 198 x 48 points, where three line-FFT launches and the
+// potential's took 38 and 102 us. The axes' radices go up to 22 here: with a whole CU's registers for one workgroup a
+// thread has 256, and 512 threads are two lines or more a thread at these sizes.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void specular_plane_kernel(cx<double>* spec, ZrShape shape, const cx<double>* table_z,
+                                                                 const cx<double>* table_r, const cx<double>* factor,
+                                                                 int potential, int nzpot, const cx<double>* gas,
+                                                                 const double* z_opt, const double* r_opt, int r_first,
+                                                                 int r_last) {
+  zr_transform<double, ZrRunTime<22>, THREADS>(
+      spec, shape, table_z, table_r, factor, nullptr, nullptr, nullptr, -1, [&](int iz, int ir, cx<double> v) {
+        if (potential) {
+          if (iz >= nzpot) v = gas[ir] * v;
+          v = scale(v, z_opt[iz]);
+          if (ir >= r_first && ir <= r_last) v = scale(v, r_opt[ir]);
+        }
+        spec[iz * shape.nr + ir] = v;
+      });
 }
 
 // Place (kz place, kr place) of the plane after the forward passes -> its entry (kz, kr) of the (iz, ir) factor.

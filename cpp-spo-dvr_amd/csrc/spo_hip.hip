@@ -217,6 +217,11 @@ struct DevicePlan {
 unsigned blocks_for(long n, int threads) { return static_cast<unsigned>((n + threads - 1) / threads); }
 
 constexpr int kThreads = 256;
+// From this many grid points on, the specular step runs on a stream of its own beside T_Zr and T_xy; below, before them
+// on their stream. The two events that join the streams cost about 18 us a block and one workgroup's step 11 us (2048
+// points), 20 (4200), 26 (6144) to 32 us (9504): on one stream 34 us a block instead of 46 (2048 points), 92 instead of
+// 97 (4200), but 369 instead of 360 (6144) and 166 instead of 145 (9504).
+constexpr int kSpecularBesidePoints = 5120;
 
 void set_lds(const void* kernel, std::size_t bytes) {
   HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
@@ -331,9 +336,16 @@ struct spo_hip_backend {
   virtual void z_plane(int iz) = 0;
   virtual void block_densities() = 0;
   virtual void site_column(int ixy, double* out) = 0;
-  virtual void bk_scattering() = 0;
+  // Every BK coefficient; from_specular: the initial state's from the specular wave at line iz_specular.
+  virtual void bk_scattering(bool from_specular, int iz_specular) = 0;
   // One analysis step of the energy-resolved sums of the scattering wave (er_phase holds exp(i E t)).
   virtual void energy_resolved_scattering() = 0;
+
+  // The specular grid's step in one launch (specular_plane_kernel), whose order the factors then have.
+  const void* spec_fn = nullptr;
+  spo_dev::ZrShape spec_shape = {};
+  std::size_t spec_lds = 0;
+  bool spec_beside = true;  // the specular step runs on `side`, beside T_Zr and T_xy
 
   // Energy-resolved sums: device layout [site][energy][irot][izr] and [energy][iz][ir].
   Buffer er_sums, er_specular, er_sites, er_phase;
@@ -348,7 +360,8 @@ struct spo_hip_backend {
 
 void spo_hip_backend::lines_d(cx<double>* data, spo_dev::Lines L, const DevicePlan<double>& p, int sign, int mode,
                               const cx<double>* factor, int f_line, int f_elem) {
-  L.lines_per_block = std::max(1, std::min(64, 65536 / (L.n * static_cast<int>(sizeof(cx<double>)))));
+  // Few lines a workgroup: the grid has a few hundred lines in all, and they should be on many CUs.
+  L.lines_per_block = std::max(1, std::min({64, 65536 / (L.n * static_cast<int>(sizeof(cx<double>))), L.count / 64}));
   const std::size_t lds = std::size_t(L.lines_per_block) * L.n * sizeof(cx<double>);
   const unsigned grid = blocks_for(L.count, L.lines_per_block);
   timed("specular_lines_fft", [&] {
@@ -361,9 +374,27 @@ void spo_hip_backend::lines_d(cx<double>* data, spo_dev::Lines L, const DevicePl
 // beyond zasymp and the absorbers (src/propagation/specular_operator.cpp:40-71). FP64.
 void spo_hip_backend::specular_step(bool half, bool kinetic_only) {
   // On `side`, after everything already on `stream` (the last projection wrote the specular wave).
-  HIP_CHECK(hipEventRecord(main_ready, stream));
-  HIP_CHECK(hipStreamWaitEvent(side, main_ready, 0));
+  const hipStream_t on = spec_beside ? side : stream;
+  if (spec_beside) {
+    HIP_CHECK(hipEventRecord(main_ready, stream));
+    HIP_CHECK(hipStreamWaitEvent(side, main_ready, 0));
+  }
   cx<double>* sp = spec.as<cx<double>>();
+  if (spec_fn) {
+    const cx<double>* tz = plan_zsp->tw();
+    const cx<double>* tr = plan_r_d->tw();
+    const cx<double>* factor = (half ? spec_half : spec_full).as<cx<double>>();
+    int potential = kinetic_only ? 0 : 1;
+    const cx<double>* gas = spec_gas.as<cx<double>>();
+    const double* zo = z_spec_opt.as<double>();
+    const double* ro = r_opt_d.as<double>();
+    void* args[] = {&sp, &spec_shape, const_cast<cx<double>**>(&tz), const_cast<cx<double>**>(&tr),
+                    const_cast<cx<double>**>(&factor), &potential, &s.nzpot, const_cast<cx<double>**>(&gas),
+                    const_cast<double**>(&zo), const_cast<double**>(&ro), &s.r_abs_first, &s.r_abs_last};
+    timed("specular_plane", [&] { launch(spec_fn, 1, spo_dev::kSpecularThreads, spec_lds, on, args); }, on);
+    if (spec_beside) HIP_CHECK(hipEventRecord(spec_ready, side));
+    return;
+  }
   spo_dev::Lines r_lines{s.nr, s.nzsp, s.nzsp, s.nr, 0, 1, 1};
   spo_dev::Lines z_lines{s.nzsp, s.nr, s.nr, 1, 0, s.nr, 1};
   lines_d(sp, r_lines, *plan_r_d, -1, 0, nullptr, 0, 0);
@@ -382,19 +413,9 @@ void spo_hip_backend::specular_step(bool half, bool kinetic_only) {
 void spo_hip_backend::analyse(int surface_fixed, int iz_specular, double t, double* coefficients) {
   const spo_hip_analysis& a = analysis;
   const std::size_t n = std::size_t(a.n_states) * a.n_v;
-  timed("bk_zero", [&] {
-    hipLaunchKernelGGL(spo_dev::zero_kernel, dim3(blocks_for(long(n), kThreads)), dim3(kThreads), 0, stream,
-                       bk.as<cx<double>>(), long(n));
-  });
-  bk_scattering();
-  if (surface_fixed) {
-    if (iz_specular < 0 || iz_specular >= s.nzsp) throw Status(SPO_HIP_E_ARGUMENT, "specular line out of range");
-    timed("bk_specular", [&] {
-      hipLaunchKernelGGL(spo_dev::bk_specular_kernel, dim3(1), dim3(64), 0, stream, spec.as<cx<double>>(), s.nr,
-                         iz_specular, a.n_v, a.n_states, a.initial_state, initial_radial.as<double>(), a.dr,
-                         bk.as<cx<double>>());
-    });
-  }
+  if (surface_fixed && (iz_specular < 0 || iz_specular >= s.nzsp))
+    throw Status(SPO_HIP_E_ARGUMENT, "specular line out of range");
+  bk_scattering(surface_fixed != 0, iz_specular);
   const long total = long(n) * a.n_energies;
   timed("s_accumulate", [&] {
     hipLaunchKernelGGL(spo_dev::s_accumulate_kernel, dim3(blocks_for(total, kThreads)), dim3(kThreads), 0, stream,
@@ -456,7 +477,7 @@ struct State final : spo_hip_backend {
   void z_plane(int iz) override;
   void block_densities() override;
   void site_column(int ixy, double* out) override;
-  void bk_scattering() override;
+  void bk_scattering(bool from_specular, int iz_specular) override;
   void energy_resolved_scattering() override;
   void lines(cx<T>* data, spo_dev::Lines L, const DevicePlan<T>& p, int sign, int mode, const cx<T>* factor,
              const cx<T>* factor_lo, int f_line, int f_elem);
@@ -849,7 +870,7 @@ void State<T>::step_block(bool specular_half, int scattering, bool kinetic_only)
   if (scattering != 0) scattering_kinetic(scattering == 1, kinetic_only);
   cx<T>* ps = psi.as<cx<T>>();
   // The specular step (on `side`) is complete before the specular wave is read or written on `stream` again.
-  HIP_CHECK(hipStreamWaitEvent(stream, spec_ready, 0));
+  if (spec_beside) HIP_CHECK(hipStreamWaitEvent(stream, spec_ready, 0));
   if (kinetic_only || s.n_zr_pot == 0) return;
   // V in the interaction region, then the projection onto the specular grid.
   spo_dev::AngularTables at{legendre.as<double>(),  block_first.as<int>(), block_size.as<int>(),
@@ -969,7 +990,7 @@ void State<T>::site_column(int ixy, double* out) {
 }
 
 template <typename T>
-void State<T>::bk_scattering() {
+void State<T>::bk_scattering(bool from_specular, int iz_specular) {
   const spo_hip_analysis& a = analysis;
   const cx<T>* src = psi.as<cx<T>>();
   spo_dev::Shape sh = s;
@@ -994,7 +1015,9 @@ void State<T>::bk_scattering() {
                        std::size_t(s.n_xy) * sizeof(cx<double>), stream, src, sh, iz,
                        a.n_rotation, a.n_diffraction, a.n_states, rot_index.as<int>(), dif_slot.as<int>(),
                        radial_weight.as<double>(), shift_f_d.as<cx<double>>(), a.xy_scale, plan_x_d->plan,
-                       plan_y_d->plan, bk.as<cx<double>>());
+                       plan_y_d->plan, bk.as<cx<double>>(),
+                       static_cast<const cx<double>*>(from_specular ? spec.as<cx<double>>() : nullptr), iz_specular,
+                       a.initial_state, initial_radial.as<double>(), a.dr);
   });
 }
 
@@ -1097,8 +1120,21 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
     zr_half_values = zh;
     const auto sf = fold(t->specular_full, std::size_t(s.nr) * s.nzsp, zr_f, sp_b);
     const auto sh = fold(t->specular_half, std::size_t(s.nr) * s.nzsp, zr_f, sp_b);
-    b->spec_full = upload(sf.data(), sf.size() * sizeof(double));
-    b->spec_half = upload(sh.data(), sh.size() * sizeof(double));
+    b->spec_lds = spo_dev::zr_plane_lds<double>(s.nzsp, s.nr);
+    if (b->spec_lds <= static_cast<std::size_t>(b->max_lds)) b->spec_fn = spo_dev::specular_plane(s.nzsp, s.nr, b->spec_shape);
+    if (b->spec_fn) set_lds(b->spec_fn, b->max_lds);  // one kernel serves grids of many sizes
+    auto specular_factor = [&](const std::vector<double>& f) {
+      if (!b->spec_fn) return upload(f.data(), f.size() * sizeof(double));
+      std::vector<double> p(f.size());
+      for (int iz = 0; iz < s.nzsp; ++iz)
+        for (int ir = 0; ir < s.nr; ++ir)
+          for (int c = 0; c < 2; ++c)
+            p[2 * (ir + std::size_t(s.nr) * iz) + c] = f[2 * spo_dev::zr_factor_order(b->spec_shape, iz, ir) + c];
+      return upload(p.data(), p.size() * sizeof(double));
+    };
+    b->spec_full = specular_factor(sf);
+    b->spec_half = specular_factor(sh);
+    b->spec_beside = !b->spec_fn || s.nzsp * s.nr >= kSpecularBesidePoints;
     const auto xf = fold(t->xy_full, s.n_xy, xy_f, xy_b), xh = fold(t->xy_half, s.n_xy, xy_f, xy_b);
     b->xy_full = upload_complex<T>(xf.data(), s.n_xy);
     b->xy_full_lo = factor_lo<T>(xf.data(), s.n_xy);

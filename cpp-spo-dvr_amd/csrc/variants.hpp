@@ -27,6 +27,10 @@ struct Variant {
 // T_Zr of a whole plane in LDS; empty for an axis that is not a product of two radices.
 template <typename T>
 std::vector<Variant> zr_variants(int nz, int nr);
+// specular_plane_kernel for a grid of this shape (its radices to shape), or NULL where an axis is not a product of two
+// radices.
+constexpr int kSpecularThreads = 512;
+const void* specular_plane(int nz, int nr, ZrShape& shape);
 template <typename T>
 std::vector<Variant> xy_reg_variants(int nx, int ny);
 // fused: the phi step in three register passes (phi_step_fused) rather than the staged LDS FFTs (8 wavefronts).

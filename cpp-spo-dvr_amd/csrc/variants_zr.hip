@@ -25,13 +25,13 @@ namespace {
   X(176, 56, 7, 8, 11, 16, 512) X(176, 56, 7, 8, 11, 16, 256) X(96, 32, 4, 8, 12, 8, 512)                      \
   X(96, 32, 4, 8, 12, 8, 256)
 
-// The two radices of an axis (first <= second, as equal as they come), or {0, 0}.
+// The two radices of an axis (first <= second <= most, as equal as they come), or {0, 0}.
 struct RadixPair {
   int low, high;
 };
-RadixPair radix_pair(int n) {
-  for (int low = 16; low >= 1; --low)
-    if (low * low <= n && n % low == 0 && register_radix(low) && register_radix(n / low)) return {low, n / low};
+RadixPair radix_pair(int n, int most = 16) {
+  for (int low = most; low >= 1; --low)
+    if (low * low <= n && n % low == 0 && register_radix(low, most) && register_radix(n / low, most)) return {low, n / low};
   return {0, 0};
 }
 
@@ -64,7 +64,7 @@ std::vector<Variant> zr_variants(int nz, int nr) {
   const RadixPair r = radix_pair(nr), z = radix_pair(nz);
   if (r.low == 0 || z.low == 0) return out;
   const ZrShape s = zr_shape(nz, nr, r.low, r.high, z.high, z.low);
-#define X(TH) out.push_back({reinterpret_cast<const void*>(zr_inplace_kernel<T, ZrRunTime, TH>), TH, TH, lds, s});
+#define X(TH) out.push_back({reinterpret_cast<const void*>(zr_inplace_kernel<T, ZrRunTime<16>, TH>), TH, TH, lds, s});
   X(256) X(512) X(1024)
 #undef X
   // Block size: the largest with which the workgroups that the planes' LDS lets onto a CU (160 KB) stay within the
@@ -78,6 +78,13 @@ std::vector<Variant> zr_variants(int nz, int nr) {
   std::stable_sort(out.begin(), out.end(),
                    [&](const Variant& a, const Variant& b) { return (a.threads == best) > (b.threads == best); });
   return out;
+}
+
+const void* specular_plane(int nz, int nr, ZrShape& shape) {
+  const RadixPair r = radix_pair(nr, 22), z = radix_pair(nz, 22);
+  if (r.low == 0 || z.low == 0) return nullptr;
+  shape = zr_shape(nz, nr, r.low, r.high, z.high, z.low);
+  return reinterpret_cast<const void*>(specular_plane_kernel<kSpecularThreads>);
 }
 
 template std::vector<Variant> zr_variants<double>(int, int);

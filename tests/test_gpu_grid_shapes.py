@@ -58,6 +58,16 @@ def test_zr_plane_shapes(nz, nr):
     _check(f"zr_{nz}_{nr}", _grid(nz, nr, 4, 2), 100 + nz + nr, blocks=((False, False), (True, True)))
 
 
+# Specular grids (NZSpecular, NR) on both sides of each choice: in one launch, with small radices and with 18, 20 and 22
+# along Z, before the scattering wave's step (up to 5120 points) and beside it; no product of two radices (420), and
+# more points than a CU's LDS holds (360 x 36), which take the line transforms.
+@pytest.mark.parametrize("nzsp,nr", [(30, 10), (198, 12), (360, 12), (396, 12), (440, 12), (308, 24), (420, 12), (360, 36)])
+def test_specular_grids(nzsp, nr):
+    p = _grid(22, nr, 4, 2)
+    p.update(Title=f"specular {nzsp} x {nr}", nZSpecular=nzsp, ZSpOptEnd=-1.0 + p["dZ"] * (nzsp - 1))
+    _check(f"sp_{nzsp}_{nr}", p, 400 + nzsp + nr, blocks=((False, False), (True, True)))
+
+
 # Every (x, y) line length of the register kernel, with izr counts that leave a partial tile, and one beyond it.
 @pytest.mark.parametrize("nxy", [2, 6, 10, 12, 14, 18])
 @pytest.mark.parametrize("nz,nr", [(22, 10), (28, 12)])

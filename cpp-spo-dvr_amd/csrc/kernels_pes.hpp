@@ -123,29 +123,31 @@ struct PesGrid {
   ScmDev scm;  // pes == 3 with a distorted slab (scm.on)
 };
 
-// One value per thread, in the table's own order: index = iphi + n_phi (itheta + n_theta (irep + n_rep izr)).
-__global__ __launch_bounds__(256) void potential_grid_kernel(PesGrid g, double* values) {
-  const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-  const long n_tp = static_cast<long>(g.n_theta) * g.n_phi;
-  if (i >= n_tp * g.n_rep * g.n_zr) return;
-  const int ip = static_cast<int>(i % g.n_phi);
-  const int it = static_cast<int>((i / g.n_phi) % g.n_theta);
-  const int irep = static_cast<int>((i / n_tp) % g.n_rep);
-  const int izr = static_cast<int>(i / (n_tp * g.n_rep));
-  const int iz = izr / g.nr, ir = izr % g.nr;
-  const int ixy = g.representatives[irep];
-  const int ix = ixy / g.ny, iy = ixy % g.ny;
-  const double z = g.z[iz];
+// A value's place in the table: index = iphi + n_phi (itheta + n_theta (irep + n_rep izr)).
+struct PesPlace {
+  int ix, iy, iz, ir, itheta, iphi;
+  __device__ PesPlace(const PesGrid& g, long i) {
+    const long n_tp = static_cast<long>(g.n_theta) * g.n_phi;
+    iphi = static_cast<int>(i % g.n_phi);
+    itheta = static_cast<int>((i / g.n_phi) % g.n_theta);
+    const int irep = static_cast<int>((i / n_tp) % g.n_rep);
+    const int izr = static_cast<int>(i / (n_tp * g.n_rep));
+    iz = izr / g.nr;
+    ir = izr % g.nr;
+    const int ixy = g.representatives[irep];
+    ix = ixy / g.ny;
+    iy = ixy % g.ny;
+  }
+};
+
+// The table's value from the surface's (eV) at Z index iz, r index ir: hartree, the switch and the limits.
+__device__ __forceinline__ double pes_grid_value(const PesGrid& g, double ev, int iz, int ir) {
   // eV -> hartree by a multiplication with 1 / 27.2114, as the reference's grid builder does
-  const double ev = g.pes == 3 ? crp_scm_qd(g.crp, g.scm, g.x[ix], g.y[iy], z, g.r[ir], g.theta[it], g.phi[ip])
-                               : pes_value(g.pes, g.x[ix], g.y[iy], z, g.r[ir], g.theta[it], g.phi[ip]);
   double v = ev * (1.0 / kHartreeInEv);
   // A point the surface cannot evaluate (NaN) stays NaN through the switch and the limits, so that the entry point
   // refuses the grid where the host build stops, also above ZmaxSwitch.
-  if (isnan(v)) {
-    values[i] = v;
-    return;
-  }
+  if (isnan(v)) return v;
+  const double z = g.z[iz];
   if (g.use_switching && tol_gt(z, g.z_min_switch)) {
     const double va = g.gas_phase[ir];
     if (tol_ge(z, g.z_max_switch)) {
@@ -157,7 +159,32 @@ __global__ __launch_bounds__(256) void potential_grid_kernel(PesGrid g, double* 
   }
   if (g.impose_v_min && v < g.v_min) v = g.v_min;
   if (g.impose_v_max && v > g.v_max) v = g.v_max;
-  values[i] = v;
+  return v;
+}
+
+// One value per thread, in the table's own order (the analytic surfaces).
+__global__ __launch_bounds__(256) void potential_grid_kernel(PesGrid g, double* values) {
+  const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= static_cast<long>(g.n_theta) * g.n_phi * g.n_rep * g.n_zr) return;
+  const PesPlace at(g, i);
+  values[i] = pes_grid_value(
+      g, pes_value(g.pes, g.x[at.ix], g.y[at.iy], g.z[at.iz], g.r[at.ir], g.theta[at.itheta], g.phi[at.iphi]), at.iz, at.ir);
+}
+
+// The same for the CRP surface, from value `first` on, n in all, 64 a workgroup.
+template <int WAVES, bool STAGED>
+__global__ __launch_bounds__(64 * WAVES, 4) void crp_grid_kernel(long first, long n, PesGrid g, double* values) {
+  const long i = first + static_cast<long>(blockIdx.x) * 64 + (threadIdx.x & 63);
+  const PesPlace at(g, i < n ? i : n - 1);
+  const double ev = crp_scm_block<WAVES, STAGED>(g.crp, g.scm, [&](double* p) {
+    p[0] = g.x[at.ix];
+    p[1] = g.y[at.iy];
+    p[2] = g.z[at.iz];
+    p[3] = g.r[at.ir];
+    p[4] = g.theta[at.itheta];
+    p[5] = g.phi[at.iphi];
+  });
+  if (threadIdx.x < 64 && i < n) values[i] = pes_grid_value(g, ev, at.iz, at.ir);
 }
 
 }  // namespace spo_dev

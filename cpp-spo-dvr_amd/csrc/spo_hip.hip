@@ -2176,6 +2176,36 @@ struct ScmUpload {
   }
 };
 
+using CrpPointsKernel = decltype(&spo_dev::crp_points_kernel<8, true>);
+constexpr CrpPointsKernel kCrpPointsKernels[2][2] = {
+    {spo_dev::crp_points_kernel<spo_dev::kCrpWaves, false>, spo_dev::crp_points_kernel<spo_dev::kCrpWaves, true>},
+    {spo_dev::crp_points_kernel<spo_dev::kCrpWavesFew, false>, spo_dev::crp_points_kernel<spo_dev::kCrpWavesFew, true>}};
+using CrpGridKernel = decltype(&spo_dev::crp_grid_kernel<8, true>);
+constexpr CrpGridKernel kCrpGridKernels[2][2] = {
+    {spo_dev::crp_grid_kernel<spo_dev::kCrpWaves, false>, spo_dev::crp_grid_kernel<spo_dev::kCrpWaves, true>},
+    {spo_dev::crp_grid_kernel<spo_dev::kCrpWavesFew, false>, spo_dev::crp_grid_kernel<spo_dev::kCrpWavesFew, true>}};
+
+// A CRP kernel over n points, 64 a workgroup: kernels[few][staged], few workgroups (at most one a CU) of 16 wavefronts
+// and the corrugation function in LDS or read from memory.
+template <class... P, class... A>
+void launch_crp(const spo_dev::CrpDev& s, void (*const (&kernels)[2][2])(long, long, P...), long n, const A&... args) {
+  int dev = 0, units = 0;
+  HIP_CHECK(hipGetDevice(&dev));
+  HIP_CHECK(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev));
+  const bool few = n <= 64L * units;
+  const bool staged = spo_dev::crp_staged_doubles(s.n_corrugation) <= spo_dev::kCrpStagedMax;
+  const auto kernel = kernels[few][staged];
+  const int threads = 64 * (few ? spo_dev::kCrpWavesFew : spo_dev::kCrpWaves);
+  const std::size_t lds = spo_dev::crp_lds(s.n_corrugation, staged);
+  set_lds(reinterpret_cast<const void*>(kernel), lds);
+  constexpr long kLaunch = 1L << 28;  // a launch has at most 2^32 threads, 8 a point here
+  for (long first = 0; first < n; first += kLaunch) {
+    const dim3 grid(blocks_for(std::min(n - first, kLaunch), 64));
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, nullptr, first, n, args...);
+    HIP_CHECK(hipGetLastError());
+  }
+}
+
 void check_finite(const double* v, long n, const char* where) {
   for (long i = 0; i < n; ++i)
     if (std::isnan(v[i]))
@@ -2202,9 +2232,7 @@ int spo_hip_scm_values(const spo_hip_crp_surface* surface, const spo_hip_scm_cor
     ScmUpload correction(scm);
     Buffer p = upload(points, std::size_t(n) * 6 * sizeof(double));
     Buffer out(std::size_t(n) * sizeof(double));
-    hipLaunchKernelGGL(spo_dev::crp_points_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, nullptr, crp.view,
-                       correction.view, n, p.as<double>(), out.as<double>());
-    HIP_CHECK(hipGetLastError());
+    launch_crp(crp.view, kCrpPointsKernels, n, crp.view, correction.view, p.as<const double>(), out.as<double>());
     HIP_CHECK(hipMemcpy(values, out.as<void>(), std::size_t(n) * sizeof(double), hipMemcpyDeviceToHost));
     check_finite(values, n, "spo_hip_crp_values");
   });
@@ -2245,9 +2273,13 @@ int spo_hip_potential_grid(const spo_hip_pes_grid* grid, double* values) {
                        ph.as<double>(), reps.as<int>(), g.use_switching, g.z_min_switch, g.z_max_switch,
                        g.use_switching ? gas.as<double>() : nullptr, g.impose_v_min, g.impose_v_max, g.v_min,
                        g.v_max, crp ? crp->view : spo_dev::CrpDev{}, correction.view};
-    hipLaunchKernelGGL(spo_dev::potential_grid_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, nullptr, d,
-                       out.as<double>());
-    HIP_CHECK(hipGetLastError());
+    if (g.pes == SPO_HIP_PES_CRP) {
+      launch_crp(d.crp, kCrpGridKernels, n, d, out.as<double>());
+    } else {
+      hipLaunchKernelGGL(spo_dev::potential_grid_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, nullptr, d,
+                         out.as<double>());
+      HIP_CHECK(hipGetLastError());
+    }
     HIP_CHECK(hipMemcpy(values, out.as<void>(), std::size_t(n) * sizeof(double), hipMemcpyDeviceToHost));
     if (g.pes == SPO_HIP_PES_CRP) check_finite(values, n, "spo_hip_potential_grid");
   });

@@ -1,0 +1,49 @@
+"""The CRP kernels at the sizes where they change: a lane, a workgroup's 64 points and one more, the last count that
+takes a workgroup a CU and the first beyond it (64 x 256 points), and a corrugation function short enough for LDS or
+longer. Against the host restatement, to the bar of test_gpu_crp.py (the same statements; the device's sin / cos and the
+sums in runs leave a few ulp of the terms)."""
+
+import os
+import shutil
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_crp import CRP_DIR, FLOOR_EV, TOL, _note, _points, _relative
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(directory, counts, seed):
+    import spodvr_amd
+    s = spodvr_amd.CrpSurface(directory)
+    try:
+        pts = _points(s, max(counts), seed)
+        host = s.qd(pts)
+        for n in counts:
+            _note("values of", n, "points, seed", seed)
+            assert _relative(s.device_qd(pts[:n]), host[:n], FLOOR_EV) <= TOL
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("case", ["cu111_srp48", "c6v_pairwise", "c4v_pairwise"])
+def test_point_counts(case):
+    _check(os.path.join(CRP_DIR, case, "dataset"), [1, 63, 64, 65, 1000, 16384, 16385], 21)
+
+
+@pytest.mark.parametrize("case", ["cu111_srp48", "c4v_pairwise"])
+@pytest.mark.parametrize("knots", [128, 129, 178, 179, 400])
+def test_corrugation_knots(case, knots, tmp_path):
+    """The data set's corrugation function resampled to `knots` points, ends and slopes kept."""
+    where = tmp_path / "dataset"
+    shutil.copytree(os.path.join(CRP_DIR, case, "dataset"), where)
+    table = where / "Atom" / "intrep.dat"
+    lines = [line for line in table.read_text().splitlines() if line.strip()]
+    count = 2  # after the slopes at both ends
+    n = int(lines[count].split()[0])
+    x, f = np.array([[float(v) for v in line.split()[:2]] for line in lines[count + 1:count + 1 + n]]).T
+    fine = np.linspace(x[0], x[-1], knots)
+    table.write_text("\n".join(lines[:count] + [str(knots)] + [f"{a:.16e} {b:.16e}" for a, b in
+                                                                zip(fine, np.interp(fine, x, f))]) + "\n")
+    _check(str(where), [500, 17000], 22)

@@ -224,7 +224,8 @@ __device__ inline double crp_staged_splint(const CrpStaged& c, double t) {
   const double h = i[1] - i[0];
   const double a = crp_quotient(i[1] - t, h, i[6]);
   const double b = crp_quotient(t - i[0], h, i[6]);
-  return a * i[2] + b * i[3] + crp_quotient(((a * a * a - a) * i[4] + (b * b * b - b) * i[5]) * (h * h), 6.0, 1.0 / 6.0);
+  const double bend = ((a * a * a - a) * i[4] + (b * b * b - b) * i[5]) * (h * h);
+  return a * i[2] + b * i[3] + crp_quotient(bend, 6.0, 1.0 / 6.0);
 }
 
 // The corrugation function summed over the cluster's atoms [first, last) (MURII, MURO / VREP1D values); NaN where the
@@ -272,7 +273,8 @@ struct CrpSite {
   int mid, reversed;
 };
 constexpr int kCrpTop = 0, kCrpBridge = 1, kCrpHollow = 2, kCrpT2 = 3;
-constexpr double kCrpPi = spo::crp_tables::kPi, kCrpPi3 = kCrpPi / 3.00, kCrp2Pi3 = 2.00 * kCrpPi3, kCrpPi6 = kCrpPi / 6.00;
+constexpr double kCrpPi = spo::crp_tables::kPi, kCrpPi3 = kCrpPi / 3.00, kCrp2Pi3 = 2.00 * kCrpPi3;
+constexpr double kCrpPi6 = kCrpPi / 6.00;
 __constant__ CrpSite kCrpSites[2][12] = {
     {{kCrpTop, 0, 0, 0, 0, 0}, {kCrpBridge, 3, 0, 0, 0, 0}, {kCrpHollow, 7, 0, 0, 0, 0}, {kCrpT2, 12, 0, kCrpPi6, 5, 0},
      {kCrpBridge, 3, kCrpPi3, 0, 0, 0}, {kCrpBridge, 3, -kCrpPi3, 0, 0, 0}, {kCrpT2, 12, -kCrp2Pi3, kCrpPi6, 5, 0},
@@ -299,7 +301,8 @@ __device__ inline double crp_site(const CrpSite& site, double phi, double c2t, d
   if (site.kind == kCrpBridge) {
     constexpr double u3 = 1.00 / 3.00;
     const double c3 = cut(3);
-    const double v90 = (c1 + 2.00 * c2) * u3 - 0.500 * (c3 - c1) * t1 + (0.500 * (c3 - c1) - 2.00 * (c2 - c1) * u3) * t2;
+    const double v90 =
+        (c1 + 2.00 * c2) * u3 - 0.500 * (c3 - c1) * t1 + (0.500 * (c3 - c1) - 2.00 * (c2 - c1) * u3) * t2;
     return 0.500 * (c0 * (1.00 + c2t) + v90 * (1.00 - c2t));
   }
   if (site.kind == kCrpHollow) {
@@ -573,7 +576,8 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
     double x = 0.0, y = 0.0, rep = 0.0;
     if (!gas_phase && !(s.square && pz >= s.cell[10 + s.cell_nz - 1])) {
       rep = crp_fold(s, px, py, x, y)
-                ? crp_cluster<STAGED>(s, staged, x, y, pz, 2 * part * s.n_cluster / WAVES, 2 * (part + 1) * s.n_cluster / WAVES)
+                ? crp_cluster<STAGED>(s, staged, x, y, pz, 2 * part * s.n_cluster / WAVES,
+                                      2 * (part + 1) * s.n_cluster / WAVES)
                 : __builtin_nan("");
     }
     slot(kCrpRep + wave) = rep;
@@ -637,7 +641,8 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
     if (wave < 2) {
       const double px = slot(kCrpA + 3 * wave), py = slot(kCrpA + 3 * wave + 1), pz = slot(kCrpA + 3 * wave + 2);
       double x = 0.0, y = 0.0, cell = 0.0;  // 0 above the data
-      if (!(pz >= s.cell[10 + s.cell_nz - 1])) cell = crp_fold(s, px, py, x, y) ? crp_cell(s, x, y, pz) : __builtin_nan("");
+      if (!(pz >= s.cell[10 + s.cell_nz - 1]))
+        cell = crp_fold(s, px, py, x, y) ? crp_cell(s, x, y, pz) : __builtin_nan("");
       slot(kCrpVs + 10 * wave) = cell;
     }
   } else {
@@ -683,7 +688,8 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
     double iv = 0.00;
     if (s.square) {  // SIS8x8
       const double p1 = slot(kCrpSiteV), p2 = slot(kCrpSiteV + 1), p5 = slot(kCrpSiteV + 2), p3 = slot(kCrpSiteV + 3);
-      const double p4 = slot(kCrpSiteV + 4), p6 = slot(kCrpSiteV + 5), p7 = slot(kCrpSiteV + 6), p8 = slot(kCrpSiteV + 7);
+      const double p4 = slot(kCrpSiteV + 4), p6 = slot(kCrpSiteV + 5), p7 = slot(kCrpSiteV + 6);
+      const double p8 = slot(kCrpSiteV + 7);
       iv = 1.0 / 8.0 * (p1 + p2 + p5 + p3 + p4 + p6 + p7 + p8) * 1.0 + 1.0 / 4.0 * (p1 - p2 + p5 - p3) * cos(fac * gx) +
            1.0 / 4.0 * (p1 + p2 - p5 - p3) * cos(fac * gy) + 1.0 / 4.0 * (p4 - p6 - p7 + p8) * sin(fac * gx) +
            1.0 / 4.0 * (p4 + p6 - p7 - p8) * sin(fac * gy) +

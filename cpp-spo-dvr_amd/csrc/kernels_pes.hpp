@@ -167,8 +167,9 @@ __global__ __launch_bounds__(256) void potential_grid_kernel(PesGrid g, double* 
   const long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= static_cast<long>(g.n_theta) * g.n_phi * g.n_rep * g.n_zr) return;
   const PesPlace at(g, i);
-  values[i] = pes_grid_value(
-      g, pes_value(g.pes, g.x[at.ix], g.y[at.iy], g.z[at.iz], g.r[at.ir], g.theta[at.itheta], g.phi[at.iphi]), at.iz, at.ir);
+  const double ev =
+      pes_value(g.pes, g.x[at.ix], g.y[at.iy], g.z[at.iz], g.r[at.ir], g.theta[at.itheta], g.phi[at.iphi]);
+  values[i] = pes_grid_value(g, ev, at.iz, at.ir);
 }
 
 // The same for the CRP surface, from value `first` on, n in all, 64 a workgroup.

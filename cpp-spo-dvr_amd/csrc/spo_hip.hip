@@ -1121,7 +1121,8 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
     const auto sf = fold(t->specular_full, std::size_t(s.nr) * s.nzsp, zr_f, sp_b);
     const auto sh = fold(t->specular_half, std::size_t(s.nr) * s.nzsp, zr_f, sp_b);
     b->spec_lds = spo_dev::zr_plane_lds<double>(s.nzsp, s.nr);
-    if (b->spec_lds <= static_cast<std::size_t>(b->max_lds)) b->spec_fn = spo_dev::specular_plane(s.nzsp, s.nr, b->spec_shape);
+    if (b->spec_lds <= static_cast<std::size_t>(b->max_lds))
+      b->spec_fn = spo_dev::specular_plane(s.nzsp, s.nr, b->spec_shape);
     if (b->spec_fn) set_lds(b->spec_fn, b->max_lds);  // one kernel serves grids of many sizes
     auto specular_factor = [&](const std::vector<double>& f) {
       if (!b->spec_fn) return upload(f.data(), f.size() * sizeof(double));
@@ -2109,7 +2110,8 @@ namespace {
 
 // A packed CRP surface, checked against its own offsets, and an SCM correction (or NULL; the atoms' layers 1 or 2, a
 // positive scale) on the device, with `room` bytes after them: one allocation and one copy. An array each (10 and the
-// slab's) cost a call 13 us apiece in allocations, copies and frees: 265 us for 1000 points, of them 44 in the kernel (now 107).
+// slab's) cost a call 13 us apiece in allocations, copies and frees: 265 us for 1000 points, of them 44 in the kernel,
+// and now 107.
 struct CrpUpload {
   Buffer memory;
   spo_dev::CrpDev view{};

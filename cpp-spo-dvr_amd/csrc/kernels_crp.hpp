@@ -10,7 +10,8 @@
 // the cluster's pair terms, the slab's, the molecular cuts, the atom splines, the Fourier terms and the sites, which
 // meet in LDS. A point is some 80 000 operations, nine tenths of them pair terms, each a search and a cubic: a thread
 // that did it all needed 256 registers and 592 bytes of scratch, one wavefront a SIMD: 318 us for 1000 points and
-// 1.92 ms for 300 007 with a slab of 73 atoms (now 44 us and 0.96 ms; the operations bound it, 0.6 ms of them in all).
+// 1.92 ms for 300 007 with a slab of 73 atoms (now 44 us and 0.96 ms; the operations bound it, 0.6 ms of them in all),
+// 12.9 ms for a potential grid of 4.46 million points and 14.8 for one of 3.94 million with the slab (now 5.0 and 8.3).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -569,158 +570,162 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
   const bool gas_phase = !(gz < s.zso_max);  // the gas-phase potential alone
   const double fac = 2.00 * kPi / s.a;
 
-  // Sums over pairs: each wavefront takes one of the atoms and its part of the cluster, and its part of the slab.
-  {
-    const int h = wave & 1, part = wave >> 1;
-    const double px = slot(kCrpA + 3 * h), py = slot(kCrpA + 3 * h + 1), pz = slot(kCrpA + 3 * h + 2);
-    double x = 0.0, y = 0.0, rep = 0.0;
-    if (!gas_phase && !(s.square && pz >= s.cell[10 + s.cell_nz - 1])) {
-      rep = crp_fold(s, px, py, x, y)
-                ? crp_cluster<STAGED>(s, staged, x, y, pz, 2 * part * s.n_cluster / WAVES,
-                                      2 * (part + 1) * s.n_cluster / WAVES)
-                : __builtin_nan("");
+  // The slab's pair terms, an equal part of its atoms each.
+  if (m.on)
+    slot(kCrpDv + wave) =
+        scm_pairs(m, slot(kCrpU) + m.cos_skew * slot(kCrpV), m.sin_skew * slot(kCrpV), slot(kCrpZ), slot(kCrpRGiven),
+                  slot(kCrpSt), slot(kCrpCt), slot(kCrpSp), slot(kCrpCp), wave * m.n_atoms / WAVES,
+                  (wave + 1) * m.n_atoms / WAVES);
+  // The surface itself, unless every point is in the gas phase (the wavefronts hold the same points and agree).
+  if (__builtin_amdgcn_ballot_w64(!gas_phase) != 0) {
+    // Sums over pairs: each wavefront takes one of the atoms and its part of the cluster.
+    {
+      const int h = wave & 1, part = wave >> 1;
+      const double px = slot(kCrpA + 3 * h), py = slot(kCrpA + 3 * h + 1), pz = slot(kCrpA + 3 * h + 2);
+      double x = 0.0, y = 0.0, rep = 0.0;
+      if (!gas_phase && !(s.square && pz >= s.cell[10 + s.cell_nz - 1])) {
+        rep = crp_fold(s, px, py, x, y)
+                  ? crp_cluster<STAGED>(s, staged, x, y, pz, 2 * part * s.n_cluster / WAVES,
+                                        2 * (part + 1) * s.n_cluster / WAVES)
+                  : __builtin_nan("");
+      }
+      slot(kCrpRep + wave) = rep;
     }
-    slot(kCrpRep + wave) = rep;
-    if (m.on)
-      slot(kCrpDv + wave) =
-          scm_pairs(m, slot(kCrpU) + m.cos_skew * slot(kCrpV), m.sin_skew * slot(kCrpV), slot(kCrpZ), slot(kCrpRGiven),
-                    slot(kCrpSt), slot(kCrpCt), slot(kCrpSp), slot(kCrpCp), wave * m.n_atoms / WAVES,
-                    (wave + 1) * m.n_atoms / WAVES);
-  }
-  // The cuts at (r, Z); one cell lookup per group of cuts on the same grid.
-  {
-    int group = -1, ci = 0, cj = 0;
-    double wxa = 0, wxb = 0, wxc = 0, wxd = 0, wya = 0, wyb = 0, wyc = 0, wyd = 0;
-    for (int k = wave; k < s.n_cuts; k += WAVES) {
-      const int nr = s.cut_shape[3 * k], nzc = s.cut_shape[3 * k + 1], g = s.cut_shape[3 * k + 2];
-      const double* blk = s.cut_data + s.cut_offsets[k];
-      const double* xr = blk;
-      const double* yz = blk + nr;
-      if (g != group) {
-        if (r < xr[0] || r > xr[nr - 1] || gz < yz[0] || gz > yz[nzc - 1]) {
-          if (!gas_phase) *silent = 1;
+    // The cuts at (r, Z); one cell lookup per group of cuts on the same grid.
+    {
+      int group = -1, ci = 0, cj = 0;
+      double wxa = 0, wxb = 0, wxc = 0, wxd = 0, wya = 0, wyb = 0, wyc = 0, wyd = 0;
+      for (int k = wave; k < s.n_cuts; k += WAVES) {
+        const int nr = s.cut_shape[3 * k], nzc = s.cut_shape[3 * k + 1], g = s.cut_shape[3 * k + 2];
+        const double* blk = s.cut_data + s.cut_offsets[k];
+        const double* xr = blk;
+        const double* yz = blk + nr;
+        if (g != group) {
+          if (r < xr[0] || r > xr[nr - 1] || gz < yz[0] || gz > yz[nzc - 1]) {
+            if (!gas_phase) *silent = 1;
+          }
+          group = g;
+          ci = crp_bisect(xr, nr, r);
+          cj = crp_bisect(yz, nzc, gz);
+          const double hx = (xr[ci + 1] - xr[ci]) * (xr[ci + 1] - xr[ci]) / 6.0;
+          wxa = (xr[ci + 1] - r) / (xr[ci + 1] - xr[ci]);
+          wxb = 1.0 - wxa;
+          wxc = (wxa * wxa * wxa - wxa) * hx;
+          wxd = (wxb * wxb * wxb - wxb) * hx;
+          const double hy = (yz[cj + 1] - yz[cj]) * (yz[cj + 1] - yz[cj]) / 6.0;
+          wya = (yz[cj + 1] - gz) / (yz[cj + 1] - yz[cj]);
+          wyb = 1.0 - wya;
+          wyc = (wya * wya * wya - wya) * hy;
+          wyd = (wyb * wyb * wyb - wyb) * hy;
         }
-        group = g;
-        ci = crp_bisect(xr, nr, r);
-        cj = crp_bisect(yz, nzc, gz);
-        const double hx = (xr[ci + 1] - xr[ci]) * (xr[ci + 1] - xr[ci]) / 6.0;
-        wxa = (xr[ci + 1] - r) / (xr[ci + 1] - xr[ci]);
-        wxb = 1.0 - wxa;
-        wxc = (wxa * wxa * wxa - wxa) * hx;
-        wxd = (wxb * wxb * wxb - wxb) * hx;
-        const double hy = (yz[cj + 1] - yz[cj]) * (yz[cj + 1] - yz[cj]) / 6.0;
-        wya = (yz[cj + 1] - gz) / (yz[cj + 1] - yz[cj]);
-        wyb = 1.0 - wya;
-        wyc = (wya * wya * wya - wya) * hy;
-        wyd = (wyb * wyb * wyb - wyb) * hy;
-      }
-      const long plane = static_cast<long>(nr) * nzc;
-      const double* f = blk + nr + nzc;
-      const double* fxx = f + plane;
-      const double* fyy = fxx + plane;
-      const double* fxxyy = fyy + plane;
-      const long p00 = ci + static_cast<long>(nr) * cj, p10 = p00 + 1, p01 = p00 + nr, p11 = p01 + 1;
-      slot(kCrpCv + k) = wxa * (wya * f[p00] + wyb * f[p01] + wyc * fyy[p00] + wyd * fyy[p01]) +
-                         wxb * (wya * f[p10] + wyb * f[p11] + wyc * fyy[p10] + wyd * fyy[p11]) +
-                         wxc * (wya * fxx[p00] + wyb * fxx[p01] + wyc * fxxyy[p00] + wyd * fxxyy[p01]) +
-                         wxd * (wya * fxx[p10] + wyb * fxx[p11] + wyc * fxxyy[p10] + wyd * fxxyy[p11]);
-    }
-  }
-  if (wave == 0) {
-    const double a[3] = {slot(kCrpA), slot(kCrpA + 1), slot(kCrpA + 2)};
-    double ct = (slot(kCrpB + 2) - a[2]) / r;
-    if (ct > 1.0) ct = 1.0;
-    const double theta = acos(ct);
-    const double ddx = slot(kCrpB) - a[0], ddy = slot(kCrpB + 1) - a[1];
-    slot(kCrpPhi) = (ddx == 0.0 && ddy == 0.0) ? 0.0 : atan2(ddy, ddx);
-    slot(kCrpC2) = cos(2.00 * theta);
-    slot(kCrpS2) = sin(2.00 * theta);
-    slot(kCrpC4) = cos(4.00 * theta);
-  }
-  if (s.square) {
-    if (wave < 2) {
-      const double px = slot(kCrpA + 3 * wave), py = slot(kCrpA + 3 * wave + 1), pz = slot(kCrpA + 3 * wave + 2);
-      double x = 0.0, y = 0.0, cell = 0.0;  // 0 above the data
-      if (!(pz >= s.cell[10 + s.cell_nz - 1]))
-        cell = crp_fold(s, px, py, x, y) ? crp_cell(s, x, y, pz) : __builtin_nan("");
-      slot(kCrpVs + 10 * wave) = cell;
-    }
-  } else {
-    // The atom splines and Fourier terms, and the molecule's Fourier terms, in turn.
-    const int n_terms = s.n_basis - 1;
-    for (int k = wave; k < 2 * s.n_basis; k += WAVES) {
-      const int h = k >= s.n_basis ? 1 : 0, i = k - h * s.n_basis;
-      const int off = s.atom_offsets[i], n = s.atom_offsets[i + 1] - off;
-      const double pz = slot(kCrpA + 3 * h + 2);
-      double v = crp_dpl(s.atom_splines + 3 * off, n, pz);
-      // z within the first site's data
-      if (i == 0 && (pz < s.atom_splines[0] || pz > s.atom_splines[n - 1])) v = __builtin_nan("");
-      slot(kCrpVs + 10 * h + i) = v;
-    }
-    for (int k = wave; k < 2 * n_terms + 11; k += WAVES) {
-      const bool molecule = k >= 2 * n_terms;
-      const int h = k >= n_terms ? 1 : 0;
-      const double x = molecule ? gx : slot(kCrpA + 3 * h), y = molecule ? gy : slot(kCrpA + 3 * h + 1);
-      const double p = fac * (x - y * kUsq3), q = fac * (2.00 * y * kUsq3);
-      if (molecule)
-        slot(kCrpFb + k - 2 * n_terms) = crp_fourier(kCrpMoleculeTerms[k - 2 * n_terms], p, q);
-      else
-        slot(kCrpF + 9 * h + k - h * n_terms) = crp_fourier(kCrpAtomTerms[s.c3v ? 1 : 0][k - h * n_terms], p, q);
-    }
-  }
-  __syncthreads();
-
-  // The sites (RRINTII, RRINT).
-  {
-    const double phi = slot(kCrpPhi), c2t = slot(kCrpC2), s2t = slot(kCrpS2), c4t = slot(kCrpC4);
-    for (int k = wave; k < (s.square ? 8 : 12); k += WAVES) {
-      if (s.square) {
-        slot(kCrpSiteV + k) = crp_site_square(k, phi, c2t, s2t, c4t, [&](int c) { return slot(kCrpCv + c); });
-      } else {
-        const CrpSite& site = kCrpSites[s.c3v ? 1 : 0][k];
-        slot(kCrpSiteV + k) = crp_site(site, phi, c2t, s2t, c4t, [&](int c) { return slot(kCrpCv + site.cut + c); });
+        const long plane = static_cast<long>(nr) * nzc;
+        const double* f = blk + nr + nzc;
+        const double* fxx = f + plane;
+        const double* fyy = fxx + plane;
+        const double* fxxyy = fyy + plane;
+        const long p00 = ci + static_cast<long>(nr) * cj, p10 = p00 + 1, p01 = p00 + nr, p11 = p01 + 1;
+        slot(kCrpCv + k) = wxa * (wya * f[p00] + wyb * f[p01] + wyc * fyy[p00] + wyd * fyy[p01]) +
+                           wxb * (wya * f[p10] + wyb * f[p11] + wyc * fyy[p10] + wyd * fyy[p11]) +
+                           wxc * (wya * fxx[p00] + wyb * fxx[p01] + wyc * fxxyy[p00] + wyd * fxxyy[p01]) +
+                           wxd * (wya * fxx[p10] + wyb * fxx[p11] + wyc * fxxyy[p10] + wyd * fxxyy[p11]);
       }
     }
-  }
-  __syncthreads();
-
-  if (wave == 0) {
-    double iv = 0.00;
-    if (s.square) {  // SIS8x8
-      const double p1 = slot(kCrpSiteV), p2 = slot(kCrpSiteV + 1), p5 = slot(kCrpSiteV + 2), p3 = slot(kCrpSiteV + 3);
-      const double p4 = slot(kCrpSiteV + 4), p6 = slot(kCrpSiteV + 5), p7 = slot(kCrpSiteV + 6);
-      const double p8 = slot(kCrpSiteV + 7);
-      iv = 1.0 / 8.0 * (p1 + p2 + p5 + p3 + p4 + p6 + p7 + p8) * 1.0 + 1.0 / 4.0 * (p1 - p2 + p5 - p3) * cos(fac * gx) +
-           1.0 / 4.0 * (p1 + p2 - p5 - p3) * cos(fac * gy) + 1.0 / 4.0 * (p4 - p6 - p7 + p8) * sin(fac * gx) +
-           1.0 / 4.0 * (p4 + p6 - p7 - p8) * sin(fac * gy) +
-           1.0 / 8.0 * (p1 - p2 - p5 + p3 - p4 + p6 - p7 + p8) * cos(fac * (gx + gy)) +
-           1.0 / 8.0 * (p1 - p2 - p5 + p3 + p4 - p6 + p7 - p8) * cos(fac * (gx - gy)) +
-           1.0 / 16.0 * (p1 + p2 + p5 + p3 - p4 - p6 - p7 - p8) * (cos(fac * (2.0 * gx)) + cos(fac * (2.0 * gy)));
-    } else {  // SISII, FOUR6II
-      for (int j = 0; j < 12; ++j) {
-        double c = 0.00;
-        for (int k = 0; k < 12; ++k) c = c + kCrpMolecule[k + 12 * j] * slot(kCrpSiteV + k);
-        iv = iv + c * (j == 0 ? 1.00 : slot(kCrpFb + j - 1));
-      }
+    if (wave == 0) {
+      const double a[3] = {slot(kCrpA), slot(kCrpA + 1), slot(kCrpA + 2)};
+      double ct = (slot(kCrpB + 2) - a[2]) / r;
+      if (ct > 1.0) ct = 1.0;
+      const double theta = acos(ct);
+      const double ddx = slot(kCrpB) - a[0], ddy = slot(kCrpB + 1) - a[1];
+      slot(kCrpPhi) = (ddx == 0.0 && ddy == 0.0) ? 0.0 : atan2(ddy, ddx);
+      slot(kCrpC2) = cos(2.00 * theta);
+      slot(kCrpS2) = sin(2.00 * theta);
+      slot(kCrpC4) = cos(4.00 * theta);
     }
-    slot(kCrpIv) = iv;
-  } else if (wave < 3) {
-    // An atom's potential (ATII): the Fourier interpolation of the reduced cuts, and the cluster's sum.
-    const int h = wave - 1;
-    double v = 0.00;
     if (s.square) {
-      v = slot(kCrpVs + 10 * h);
+      if (wave < 2) {
+        const double px = slot(kCrpA + 3 * wave), py = slot(kCrpA + 3 * wave + 1), pz = slot(kCrpA + 3 * wave + 2);
+        double x = 0.0, y = 0.0, cell = 0.0;  // 0 above the data
+        if (!(pz >= s.cell[10 + s.cell_nz - 1]))
+          cell = crp_fold(s, px, py, x, y) ? crp_cell(s, x, y, pz) : __builtin_nan("");
+        slot(kCrpVs + 10 * wave) = cell;
+      }
     } else {
-      const double* coefficients = s.c3v ? kCrpAtomC3v.data() : kCrpAtomC6v.data();
-      for (int j = 0; j < s.n_basis; ++j) {
-        double a = 0.00;
-        for (int i = 0; i < s.n_basis; ++i) a = a + coefficients[i + s.n_basis * j] * slot(kCrpVs + 10 * h + i);
-        v = v + a * (j == 0 ? 1.00 : slot(kCrpF + 9 * h + j - 1));
+      // The atom splines and Fourier terms, and the molecule's Fourier terms, in turn.
+      const int n_terms = s.n_basis - 1;
+      for (int k = wave; k < 2 * s.n_basis; k += WAVES) {
+        const int h = k >= s.n_basis ? 1 : 0, i = k - h * s.n_basis;
+        const int off = s.atom_offsets[i], n = s.atom_offsets[i + 1] - off;
+        const double pz = slot(kCrpA + 3 * h + 2);
+        double v = crp_dpl(s.atom_splines + 3 * off, n, pz);
+        // z within the first site's data
+        if (i == 0 && (pz < s.atom_splines[0] || pz > s.atom_splines[n - 1])) v = __builtin_nan("");
+        slot(kCrpVs + 10 * h + i) = v;
+      }
+      for (int k = wave; k < 2 * n_terms + 11; k += WAVES) {
+        const bool molecule = k >= 2 * n_terms;
+        const int h = k >= n_terms ? 1 : 0;
+        const double x = molecule ? gx : slot(kCrpA + 3 * h), y = molecule ? gy : slot(kCrpA + 3 * h + 1);
+        const double p = fac * (x - y * kUsq3), q = fac * (2.00 * y * kUsq3);
+        if (molecule)
+          slot(kCrpFb + k - 2 * n_terms) = crp_fourier(kCrpMoleculeTerms[k - 2 * n_terms], p, q);
+        else
+          slot(kCrpF + 9 * h + k - h * n_terms) = crp_fourier(kCrpAtomTerms[s.c3v ? 1 : 0][k - h * n_terms], p, q);
       }
     }
-    double rep = slot(kCrpRep + h);
-    for (int part = 1; part < WAVES / 2; ++part) rep = rep + slot(kCrpRep + 2 * part + h);
-    slot(kCrpVa + h) = v + rep;
+    __syncthreads();
+
+    // The sites (RRINTII, RRINT).
+    {
+      const double phi = slot(kCrpPhi), c2t = slot(kCrpC2), s2t = slot(kCrpS2), c4t = slot(kCrpC4);
+      for (int k = wave; k < (s.square ? 8 : 12); k += WAVES) {
+        if (s.square) {
+          slot(kCrpSiteV + k) = crp_site_square(k, phi, c2t, s2t, c4t, [&](int c) { return slot(kCrpCv + c); });
+        } else {
+          const CrpSite& site = kCrpSites[s.c3v ? 1 : 0][k];
+          slot(kCrpSiteV + k) = crp_site(site, phi, c2t, s2t, c4t, [&](int c) { return slot(kCrpCv + site.cut + c); });
+        }
+      }
+    }
+    __syncthreads();
+
+    if (wave == 0) {
+      double iv = 0.00;
+      if (s.square) {  // SIS8x8
+        const double p1 = slot(kCrpSiteV), p2 = slot(kCrpSiteV + 1), p5 = slot(kCrpSiteV + 2), p3 = slot(kCrpSiteV + 3);
+        const double p4 = slot(kCrpSiteV + 4), p6 = slot(kCrpSiteV + 5), p7 = slot(kCrpSiteV + 6);
+        const double p8 = slot(kCrpSiteV + 7);
+        iv = 1.0 / 8.0 * (p1 + p2 + p5 + p3 + p4 + p6 + p7 + p8) * 1.0 +
+             1.0 / 4.0 * (p1 - p2 + p5 - p3) * cos(fac * gx) + 1.0 / 4.0 * (p1 + p2 - p5 - p3) * cos(fac * gy) +
+             1.0 / 4.0 * (p4 - p6 - p7 + p8) * sin(fac * gx) + 1.0 / 4.0 * (p4 + p6 - p7 - p8) * sin(fac * gy) +
+             1.0 / 8.0 * (p1 - p2 - p5 + p3 - p4 + p6 - p7 + p8) * cos(fac * (gx + gy)) +
+             1.0 / 8.0 * (p1 - p2 - p5 + p3 + p4 - p6 + p7 - p8) * cos(fac * (gx - gy)) +
+             1.0 / 16.0 * (p1 + p2 + p5 + p3 - p4 - p6 - p7 - p8) * (cos(fac * (2.0 * gx)) + cos(fac * (2.0 * gy)));
+      } else {  // SISII, FOUR6II
+        for (int j = 0; j < 12; ++j) {
+          double c = 0.00;
+          for (int k = 0; k < 12; ++k) c = c + kCrpMolecule[k + 12 * j] * slot(kCrpSiteV + k);
+          iv = iv + c * (j == 0 ? 1.00 : slot(kCrpFb + j - 1));
+        }
+      }
+      slot(kCrpIv) = iv;
+    } else if (wave < 3) {
+      // An atom's potential (ATII): the Fourier interpolation of the reduced cuts, and the cluster's sum.
+      const int h = wave - 1;
+      double v = 0.00;
+      if (s.square) {
+        v = slot(kCrpVs + 10 * h);
+      } else {
+        const double* coefficients = s.c3v ? kCrpAtomC3v.data() : kCrpAtomC6v.data();
+        for (int j = 0; j < s.n_basis; ++j) {
+          double a = 0.00;
+          for (int i = 0; i < s.n_basis; ++i) a = a + coefficients[i + s.n_basis * j] * slot(kCrpVs + 10 * h + i);
+          v = v + a * (j == 0 ? 1.00 : slot(kCrpF + 9 * h + j - 1));
+        }
+      }
+      double rep = slot(kCrpRep + h);
+      for (int part = 1; part < WAVES / 2; ++part) rep = rep + slot(kCrpRep + 2 * part + h);
+      slot(kCrpVa + h) = v + rep;
+    }
   }
   __syncthreads();
   if (wave != 0) return 0.0;

@@ -738,8 +738,8 @@ bool State<T>::build_angular_plan(const spo_hip_tables* t, const std::vector<int
 // their multiply-adds differently, so their results can differ in the last bits, and the default is therefore
 // fixed: the first variant of each family (ordered by what measured fastest on MI355X for the shape), which keeps
 // repeated runs bitwise identical. SPO_HIP_TUNE=auto makes the first backend of a process with a given shape and
-// precision time every variant on the (still zero) scattering wave, one warm-up and two timed launches each, and
-// keep the fastest for the process; SPO_HIP_TUNE="zr=384,xy=8,interaction=16" forces variants by thread count
+// precision time every variant on the scattering wave's memory (cleared afterwards), one warm-up and two timed
+// launches each, and keep the fastest for the process; SPO_HIP_TUNE="zr=384,xy=8,interaction=16" forces variants by thread count
 // (zr), izr per tile (xy) or wavefronts (interaction), and "interaction=#2" the variant at that place in the
 // family's list (variants of one size that differ in their FFT radices).
 std::map<std::string, int>& tune_cache() {
@@ -774,6 +774,7 @@ template <typename T>
 void State<T>::tune() {
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
+  bool ran = false;  // kernels ran on the scattering wave
   auto pick = [&](const std::vector<Variant>& v, const char* family, bool by_threads, auto&& run) -> int {
     if (v.size() < 2) return 0;
     const int forced = forced_variant(v, family, by_threads);
@@ -784,6 +785,7 @@ void State<T>::tune() {
                             std::to_string(dev);
     const auto hit = tune_cache().find(key);
     if (hit != tune_cache().end()) return hit->second;
+    ran = true;
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
@@ -811,10 +813,12 @@ void State<T>::tune() {
                    by_threads ? v[best].threads : v[best].param, best, v.size(), best_ms);
     return best;
   };
-  // The scattering wave is zero here, and every kernel maps zero to zero.
   zr_pick = pick(zr_variants, "zr", true, [&](const Variant& v) { run_zr(v, false); });
   xy_pick = pick(xy_variants, "xy", false, [&](const Variant& v) { run_xy(v, false, false); });
   v_pick = pick(v_variants, "interaction", false, [&](const Variant& v) { run_interaction(v); });
+  // The interaction adds the specular wave's part to the scattering wave, which is zero again when this returns.
+  if (ran)
+    HIP_CHECK(hipMemsetAsync(psi.as<void>(), 0, std::size_t(s.n_zr) * s.n_rot * s.n_xy * sizeof(cx<T>), stream));
   HIP_CHECK(hipStreamSynchronize(stream));
 }
 

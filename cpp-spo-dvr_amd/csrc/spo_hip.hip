@@ -734,16 +734,21 @@ bool State<T>::build_angular_plan(const spo_hip_tables* t, const std::vector<int
   return true;
 }
 
-// The launch tuner. The variants of one family differ only in block sizes and tiles; the compiler may contract
-// their multiply-adds differently, so their results can differ in the last bits, and the default is therefore
+// The launch tuner. The variants of one family compute the same transforms with other block sizes, tiles and FFT
+// radices (interaction: in other kernels), so their results can differ in the last bits, and the default is therefore
 // fixed: the first variant of each family (ordered by what measured fastest on MI355X for the shape), which keeps
-// repeated runs bitwise identical. SPO_HIP_TUNE=auto makes the first backend of a process with a given shape and
-// precision time every variant on the scattering wave's memory (cleared afterwards), one warm-up and two timed
-// launches each, and keep the fastest for the process; SPO_HIP_TUNE="zr=384,xy=8,interaction=16" forces variants by thread count
-// (zr), izr per tile (xy) or wavefronts (interaction), and "interaction=#2" the variant at that place in the
-// family's list (variants of one size that differ in their FFT radices).
-std::map<std::string, int>& tune_cache() {
-  static std::map<std::string, int> cache;
+// repeated runs bitwise identical. SPO_HIP_TUNE=auto makes the first backend of a process with a given shape, precision
+// and list of variants time every one on the scattering wave's memory (cleared afterwards), one warm-up and two timed
+// launches each, and keep the fastest for the process. The list belongs to the key because its order and length depend
+// on more than the shape: the tables, SPO_HIP_INTERACTION and SPO_HIP_CONTRACTION. SPO_HIP_TUNE="zr=384,xy=8,
+// interaction=16" forces variants by thread count (zr), izr per tile (xy) or wavefronts (interaction), and
+// "interaction=#2" the variant at that place in the family's list (0 = the default).
+struct TuneCache {
+  std::mutex mutex;
+  std::map<std::string, int> picks;  // shape and list -> place in that list
+};
+TuneCache& tune_cache() {
+  static TuneCache cache;
   return cache;
 }
 
@@ -779,12 +784,18 @@ void State<T>::tune() {
     if (v.size() < 2) return 0;
     const int forced = forced_variant(v, family, by_threads);
     if (forced >= 0) return forced;
-    const std::string key = std::string(family) + ":" + std::to_string(s.nz) + "x" + std::to_string(s.nr) + "x" +
-                            std::to_string(s.nx) + "x" + std::to_string(s.ny) + "x" + std::to_string(s.n_rot) +
-                            "x" + std::to_string(s.n_phi) + ":" + std::to_string(sizeof(T)) + ":" +
-                            std::to_string(dev);
-    const auto hit = tune_cache().find(key);
-    if (hit != tune_cache().end()) return hit->second;
+    std::string key = std::string(family) + ":";
+    for (int n : {s.nz, s.nr, s.nx, s.ny, s.nzpot, s.n_rot, s.n_theta, s.n_phi, s.n_rep}) key += std::to_string(n) + "x";
+    key.back() = ':';
+    key += std::to_string(sizeof(T)) + ":" + std::to_string(dev);
+    std::string list = key;
+    for (const Variant& one : v)
+      list += ":" + std::to_string(reinterpret_cast<std::uintptr_t>(one.fn)) + "/" + std::to_string(one.threads);
+    {
+      const std::lock_guard<std::mutex> lock(tune_cache().mutex);
+      const auto hit = tune_cache().picks.find(list);
+      if (hit != tune_cache().picks.end()) return hit->second;
+    }
     ran = true;
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
@@ -807,7 +818,10 @@ void State<T>::tune() {
     }
     HIP_CHECK(hipEventDestroy(e0));
     HIP_CHECK(hipEventDestroy(e1));
-    tune_cache()[key] = best;
+    {
+      const std::lock_guard<std::mutex> lock(tune_cache().mutex);
+      tune_cache().picks[list] = best;
+    }
     if (std::getenv("SPO_HIP_TUNE_LOG"))
       std::fprintf(stderr, "spo_hip tune %s: %s=%d (#%d of %zu, %.3f ms for two launches)\n", key.c_str(), family,
                    by_threads ? v[best].threads : v[best].param, best, v.size(), best_ms);

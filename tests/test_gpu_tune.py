@@ -57,3 +57,33 @@ def test_a_tuned_run_starts_from_an_empty_scattering_wave(case, precision):
             assert relative_difference(want, tuned.bk_records()) < (1e-12 if precision == "fp64" else 1e-5)
         finally:
             tuned.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_variants_are_timed_for_each_shape_and_list(precision, capfd):
+    """A choice is reused by a run of the same shape with the same variants to choose from, and by no other: not where
+    the interaction region is shorter, nor where SPO_HIP_INTERACTION leaves some kernels out of the list."""
+    def timed(**overrides):
+        capfd.readouterr()
+        run = _run("dz_angular", precision, "auto", **overrides)
+        try:
+            assert np.isfinite(run.bk_records()).all()
+            run.propagate()
+            assert np.isfinite(run.get_wave()[0]).all()
+        finally:
+            run.close()
+        return sorted(line.split()[2].split(":")[0] for line in capfd.readouterr().err.splitlines()
+                      if line.startswith("spo_hip tune"))
+
+    # regions of their own, which no other test of this process has timed
+    first = {"ZmaxSwitch": 7.3}
+    assert "interaction" in timed(**first)
+    assert timed(**first) == []
+    assert "interaction" in timed(ZmaxSwitch=6.3)
+    os.environ["SPO_HIP_INTERACTION"] = "mfma"
+    try:
+        assert timed(**first) == ["interaction"]
+        assert timed(**first) == []
+    finally:
+        os.environ.pop("SPO_HIP_INTERACTION", None)
+    assert timed(**first) == []

@@ -466,6 +466,7 @@ struct State final : spo_hip_backend {
   void run_zr(const Variant& v, bool half, cx<T>* row_out = nullptr, int row = -1);
   void run_xy(const Variant& v, bool half, bool kinetic_only, cx<T>* data = nullptr,
               const spo_dev::Shape* on = nullptr);
+  void run_coupling();
   void run_interaction(const Variant& v);
   void tune();
   void scattering_kinetic(bool half, bool kinetic_only);
@@ -547,6 +548,13 @@ void State<T>::run_xy(const Variant& v, bool half, bool kinetic_only, cx<T>* dat
                   &needs_shift, &apply_potential, const_cast<T**>(&zo), const_cast<cx<T>**>(&bf),
                   const_cast<cx<T>**>(&gs), &lo};
   launch(v.fn, tiles * sh.n_rot, v.threads, v.lds, stream, args);
+}
+
+// The specular wave's part of the initial channel, ahead of an interaction kernel that does not add it itself.
+template <typename T>
+void State<T>::run_coupling() {
+  hipLaunchKernelGGL(spo_dev::specular_coupling_kernel<T>, dim3(blocks_for(long(s.n_zr_pot) * s.n_xy, 256)), dim3(256),
+                     0, stream, psi.as<cx<T>>(), spec.as<cx<double>>(), s, rot_half.as<cx<T>>(), s2sc.as<cx<T>>());
 }
 
 template <typename T>
@@ -829,7 +837,11 @@ void State<T>::tune() {
   };
   zr_pick = pick(zr_variants, "zr", true, [&](const Variant& v) { run_zr(v, false); });
   xy_pick = pick(xy_variants, "xy", false, [&](const Variant& v) { run_xy(v, false, false); });
-  v_pick = pick(v_variants, "interaction", false, [&](const Variant& v) { run_interaction(v); });
+  // Each kernel with what it needs for the same work: those that read the wave as it is, after the specular coupling.
+  v_pick = pick(v_variants, "interaction", false, [&](const Variant& v) {
+    if (v.kind != spo_dev::InteractionKind::in_place) run_coupling();
+    run_interaction(v);
+  });
   // The interaction adds the specular wave's part to the scattering wave, which is zero again when this returns.
   if (ran)
     HIP_CHECK(hipMemsetAsync(psi.as<void>(), 0, std::size_t(s.n_zr) * s.n_rot * s.n_xy * sizeof(cx<T>), stream));
@@ -902,10 +914,7 @@ void State<T>::step_block(bool specular_half, int scattering, bool kinetic_only)
   const cx<T>* ssc = s2sc.as<cx<T>>();
   if (!v_variants.empty()) {
     if (v_variants[v_pick].kind != spo_dev::InteractionKind::in_place)
-      timed("specular_coupling", [&] {
-        hipLaunchKernelGGL(spo_dev::specular_coupling_kernel<T>, dim3(blocks_for(long(s.n_zr_pot) * s.n_xy, 256)),
-                           dim3(256), 0, stream, ps, sp, s, rh, ssc);
-      });
+      timed("specular_coupling", [&] { run_coupling(); });
     timed("interaction", [&] { run_interaction(v_variants[v_pick]); });
   } else if (v_fn) {
     const cx<T>* tp = plan_phi->tw();

@@ -10,8 +10,10 @@
 // the cluster's pair terms, the slab's, the molecular cuts, the atom splines, the Fourier terms and the sites, which
 // meet in LDS. A point is some 80 000 operations, nine tenths of them pair terms, each a search and a cubic: a thread
 // that did it all needed 256 registers and 592 bytes of scratch, one wavefront a SIMD: 318 us for 1000 points and
-// 1.92 ms for 300 007 with a slab of 73 atoms (now 44 us and 0.96 ms; the operations bound it, 0.6 ms of them in all),
-// 12.9 ms for a potential grid of 4.46 million points and 14.8 for one of 3.94 million with the slab (now 5.0 and 8.3).
+// 1.92 ms for 300 007 with a slab of 73 atoms (now 43 us and 0.81 ms; the operations bound it, 0.6 ms of them in all),
+// 12.9 ms for a potential grid of 4.46 million points and 14.8 for one of 3.94 million with the slab (now 4.3 and 7.0).
+// At four wavefronts a SIMD a lane has 128 registers, and 104 to 136 bytes of its values still go to scratch, nearly all of
+// them inside the pair sums.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -427,9 +429,15 @@ __device__ inline double scm_distance(const double* a, const double* b) {
   return sqrt((dx * dx + dy * dy) + dz * dz);
 }
 
-// The pair terms of the slab's atoms [first, last) (hartree) with the molecule's centre at the Cartesian (x, y), z.
+// The sums over the cluster (both atoms') and over the slab's atoms are made in this many runs of consecutive terms,
+// whatever the number of wavefronts that share them: a point's value does not depend on the launch it is part of.
+constexpr int kCrpParts = 16;
+
+// The pair terms of the slab's atoms (hartree) with the molecule's centre at the Cartesian (x, y), z: the sums of the
+// atoms [first, mid), to `head`, and [mid, last), returned. TWO: whether the first are asked for (else mid = first).
+template <bool TWO>
 __device__ inline double scm_pairs(const ScmDev& m, double x, double y, double z, double r, double st, double ct,
-                                   double sp, double cp, int first, int last) {
+                                   double sp, double cp, int first, int mid, int last, double& head) {
   const double h = 0.5 * r;
   const double o[3] = {(h * st) * cp, (h * st) * sp, h * ct};
   double hd[2][3] = {{x - o[0], y - o[1], z - o[2]}, {x + o[0], y + o[1], z + o[2]}};
@@ -460,11 +468,19 @@ __device__ inline double scm_pairs(const ScmDev& m, double x, double y, double z
     }
   };
   for (int i = first; i < last; ++i) {
+    if (TWO && i == mid) {
+      head = dv;
+      dv = +0.0;
+    }
     const double* at = m.atoms + 7 * i;
     if (at[6] == 1.0)
       atom(t[0], at);
     else
       atom(t[1], at);
+  }
+  if (TWO && mid == last) {
+    head = dv;
+    dv = +0.0;
   }
   return dv;
 }
@@ -476,9 +492,9 @@ enum CrpSlot {
   kCrpB = kCrpA + 3,
   kCrpR = kCrpB + 3,                // their distance
   kCrpPhi, kCrpC2, kCrpS2, kCrpC4,  // the molecule's azimuth; cos 2 theta, sin 2 theta, cos 4 theta
-  kCrpRep,                          // the cluster sums, a wavefront each
-  kCrpDv = kCrpRep + kCrpWavesFew,  // the slab sums
-  kCrpCv = kCrpDv + kCrpWavesFew,   // the molecular cuts
+  kCrpRep,                          // the cluster sums, the atoms' in turn
+  kCrpDv = kCrpRep + kCrpParts,     // the slab sums
+  kCrpCv = kCrpDv + kCrpParts,      // the molecular cuts
   kCrpVs = kCrpCv + 29,             // the atom splines, 10 an atom (C4v: the cell's spline, the first of each)
   kCrpF = kCrpVs + 20,              // the atoms' Fourier terms, 9 an atom
   kCrpFb = kCrpF + 18,              // the molecule's
@@ -561,6 +577,20 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
   }
   __syncthreads();
 
+  // The slab's pair terms: each wavefront's parts of its atoms.
+  constexpr int kOwn = kCrpParts / WAVES;  // parts of a wavefront
+  static_assert(kOwn == 1 || kOwn == 2);
+  if (m.on) {
+    auto start = [&](int part) { return part * m.n_atoms / kCrpParts; };
+    double head = 0.0;
+    slot(kCrpDv + kOwn * wave + kOwn - 1) = scm_pairs<kOwn == 2>(
+        m, slot(kCrpU) + m.cos_skew * slot(kCrpV), m.sin_skew * slot(kCrpV), slot(kCrpZ), slot(kCrpRGiven), slot(kCrpSt),
+        slot(kCrpCt), slot(kCrpSp), slot(kCrpCp), start(kOwn * wave), start(kOwn * wave + kOwn - 1),
+        start(kOwn * wave + kOwn), head);
+    if (kOwn == 2) slot(kCrpDv + kOwn * wave) = head;
+  }
+
+  // Set up only now: the slab's sums need every register.
   const CrpStaged staged{table, table + crp_staged_size(s.n_corrugation), crp_staged_size(s.n_corrugation),
                          s.n_corrugation - 2};
   const double r = slot(kCrpR);
@@ -570,26 +600,25 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
   const bool gas_phase = !(gz < s.zso_max);  // the gas-phase potential alone
   const double fac = 2.00 * kPi / s.a;
 
-  // The slab's pair terms, an equal part of its atoms each.
-  if (m.on)
-    slot(kCrpDv + wave) =
-        scm_pairs(m, slot(kCrpU) + m.cos_skew * slot(kCrpV), m.sin_skew * slot(kCrpV), slot(kCrpZ), slot(kCrpRGiven),
-                  slot(kCrpSt), slot(kCrpCt), slot(kCrpSp), slot(kCrpCp), wave * m.n_atoms / WAVES,
-                  (wave + 1) * m.n_atoms / WAVES);
   // The surface itself, unless every point is in the gas phase (the wavefronts hold the same points and agree).
   if (__builtin_amdgcn_ballot_w64(!gas_phase) != 0) {
-    // Sums over pairs: each wavefront takes one of the atoms and its part of the cluster.
+    // Sums over pairs: each wavefront takes one of the atoms and its parts of the cluster.
     {
-      const int h = wave & 1, part = wave >> 1;
+      const int h = wave & 1;
       const double px = slot(kCrpA + 3 * h), py = slot(kCrpA + 3 * h + 1), pz = slot(kCrpA + 3 * h + 2);
-      double x = 0.0, y = 0.0, rep = 0.0;
-      if (!gas_phase && !(s.square && pz >= s.cell[10 + s.cell_nz - 1])) {
-        rep = crp_fold(s, px, py, x, y)
-                  ? crp_cluster<STAGED>(s, staged, x, y, pz, 2 * part * s.n_cluster / WAVES,
-                                        2 * (part + 1) * s.n_cluster / WAVES)
-                  : __builtin_nan("");
+      double x = 0.0, y = 0.0;
+      const bool in_reach = !gas_phase && !(s.square && pz >= s.cell[10 + s.cell_nz - 1]);
+      const bool folded = in_reach && crp_fold(s, px, py, x, y);
+#pragma unroll 1
+      for (int k = 0; k < kOwn; ++k) {
+        const int part = kOwn * (wave >> 1) + k;
+        double rep = 0.0;
+        if (in_reach)
+          rep = folded ? crp_cluster<STAGED>(s, staged, x, y, pz, 2 * part * s.n_cluster / kCrpParts,
+                                             2 * (part + 1) * s.n_cluster / kCrpParts)
+                       : __builtin_nan("");
+        slot(kCrpRep + 2 * part + h) = rep;
       }
-      slot(kCrpRep + wave) = rep;
     }
     // The cuts at (r, Z); one cell lookup per group of cuts on the same grid.
     {
@@ -723,7 +752,7 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
         }
       }
       double rep = slot(kCrpRep + h);
-      for (int part = 1; part < WAVES / 2; ++part) rep = rep + slot(kCrpRep + 2 * part + h);
+      for (int part = 1; part < kCrpParts / 2; ++part) rep = rep + slot(kCrpRep + 2 * part + h);
       slot(kCrpVa + h) = v + rep;
     }
   }
@@ -752,7 +781,7 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
   v = v * (1.0 * ev) - s.h2_asymptote * (1.0 * ev);
   if (m.on) {
     double dv = slot(kCrpDv);
-    for (int k = 1; k < WAVES; ++k) dv = dv + slot(kCrpDv + k);
+    for (int k = 1; k < kCrpParts; ++k) dv = dv + slot(kCrpDv + k);
     v = v + dv / 0.036749308286;
   }
   return v;
@@ -760,7 +789,7 @@ __device__ __forceinline__ double crp_scm_block(const CrpDev& s, const ScmDev& m
 
 // V at the points (u, v, Z, r, theta, phi) from `first` on, n in all, 64 a workgroup. Two workgroups of 8 wavefronts
 // share a CU, one waiting while the other works; up to a workgroup a CU, 16 wavefronts shorten the chain instead.
-// 1000 points 44 us with 16 wavefronts and 60 with 8; 300 007 with the slab 1.30 ms and 0.96.
+// 1000 points 43 us with 16 wavefronts and 60 with 8; 300 007 with the slab 1.10 ms and 0.81.
 template <int WAVES, bool STAGED>
 __global__ __launch_bounds__(64 * WAVES, 4) void crp_points_kernel(long first, long n, CrpDev s, ScmDev m,
                                                                        const double* points, double* values) {

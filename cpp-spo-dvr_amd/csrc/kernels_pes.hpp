@@ -176,16 +176,19 @@ __global__ __launch_bounds__(256) void potential_grid_kernel(PesGrid g, double* 
 template <int WAVES, bool STAGED>
 __global__ __launch_bounds__(64 * WAVES, 4) void crp_grid_kernel(long first, long n, PesGrid g, double* values) {
   const long i = first + static_cast<long>(blockIdx.x) * 64 + (threadIdx.x & 63);
-  const PesPlace at(g, i < n ? i : n - 1);
+  int iz = 0, ir = 0;  // of the first wavefront
   const double ev = crp_scm_block<WAVES, STAGED>(g.crp, g.scm, [&](double* p) {
+    const PesPlace at(g, i < n ? i : n - 1);
     p[0] = g.x[at.ix];
     p[1] = g.y[at.iy];
     p[2] = g.z[at.iz];
     p[3] = g.r[at.ir];
     p[4] = g.theta[at.itheta];
     p[5] = g.phi[at.iphi];
+    iz = at.iz;
+    ir = at.ir;
   });
-  if (threadIdx.x < 64 && i < n) values[i] = pes_grid_value(g, ev, at.iz, at.ir);
+  if (threadIdx.x < 64 && i < n) values[i] = pes_grid_value(g, ev, iz, ir);
 }
 
 }  // namespace spo_dev

@@ -9,7 +9,7 @@ import shutil
 import numpy as np
 import pytest
 
-from tests.test_gpu_crp import CRP_DIR, FLOOR_EV, TOL, _note, _points, _relative
+from tests.test_gpu_crp import CRP_DIR, FLOOR_EV, SCM_DIR, SCM_RUNS, TOL, _note, _points, _relative
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,37 @@ def test_corrugation_knots(case, knots, tmp_path):
     table.write_text("\n".join(lines[:count] + [str(knots)] + [f"{a:.16e} {b:.16e}" for a, b in
                                                                 zip(fine, np.interp(fine, x, f))]) + "\n")
     _check(str(where), [500, 17000], 22)
+
+
+@pytest.mark.parametrize("case", ["cu111_srp48", "c4v_pairwise"])
+def test_a_value_does_not_depend_on_the_points_beside_it(case):
+    """A geometry's value bit for bit the same alone, among few points and among many (the kernel's two workgroup
+    sizes)."""
+    import spodvr_amd
+    s = spodvr_amd.CrpSurface(os.path.join(CRP_DIR, case, "dataset"))
+    try:
+        pts = _points(s, 20000, 23)
+        _note("values of 20000 points and of runs of them", case)
+        many = s.device_qd(pts)
+        for n in (1, 65, 1000):
+            assert np.array_equal(s.device_qd(pts[:n]), many[:n]), n
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("run", ["example/rescaling_on", "synthetic/v3_slab3_rescaling_on"])
+def test_a_slab_value_does_not_depend_on_the_points_beside_it(run):
+    import spodvr_amd
+    f = np.load(os.path.join(SCM_DIR, run + ".npz"))
+    par, slab = SCM_RUNS[run]
+    s = spodvr_amd.ScmSurface(os.path.join(CRP_DIR, "cu111_srp48", "dataset"), os.path.join(SCM_DIR, par),
+                              os.path.join(SCM_DIR, slab), int(f["slab_number"]), float(f["cutoff"]),
+                              bool(f["rescaling"]))
+    try:
+        _note("SCM values of 20000 points and of runs of them", run)
+        pts = np.resize(f["points"], (20000, 6))
+        many = s.device_values(pts)
+        for n in (1, 65, 1000):
+            assert np.array_equal(s.device_values(pts[:n]), many[:n]), n
+    finally:
+        s.close()

@@ -504,10 +504,8 @@ enum CrpSlot {
   kCrpVa = kCrpIv + 1,
   kCrpSlots = kCrpVa + 2
 };
-// Bytes of LDS; staged: the corrugation function is in LDS too.
-inline std::size_t crp_lds(int n_corrugation, bool staged) {
-  return (64 * kCrpSlots + (staged ? crp_staged_doubles(n_corrugation) : 0)) * sizeof(double) + 64 * sizeof(int);
-}
+// Bytes of LDS, `staged` doubles of them for the corrugation function.
+constexpr std::size_t crp_lds(int staged) { return (64 * kCrpSlots + staged) * sizeof(double) + 64 * sizeof(int); }
 // Two workgroups fit on a CU with a table of this many doubles; a longer one is read from memory.
 constexpr int kCrpStagedMax = 1496;
 

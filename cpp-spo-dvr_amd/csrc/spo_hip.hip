@@ -2240,11 +2240,13 @@ void launch_crp(const spo_dev::CrpDev& s, void (*const (&kernels)[2][2])(long, l
   HIP_CHECK(hipGetDevice(&dev));
   HIP_CHECK(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev));
   const bool few = n <= 64L * units;
-  const bool staged = spo_dev::crp_staged_doubles(s.n_corrugation) <= spo_dev::kCrpStagedMax;
+  const int doubles = spo_dev::crp_staged_doubles(s.n_corrugation);
+  const bool staged = doubles <= spo_dev::kCrpStagedMax;
   const auto kernel = kernels[few][staged];
   const int threads = 64 * (few ? spo_dev::kCrpWavesFew : spo_dev::kCrpWaves);
-  const std::size_t lds = spo_dev::crp_lds(s.n_corrugation, staged);
-  set_lds(reinterpret_cast<const void*>(kernel), lds);
+  const std::size_t lds = spo_dev::crp_lds(staged ? doubles : 0);
+  // The kernel's limit is one for the process: the same for every table, so that threads with other surfaces agree.
+  set_lds(reinterpret_cast<const void*>(kernel), spo_dev::crp_lds(spo_dev::kCrpStagedMax));
   constexpr long kLaunch = 1L << 28;  // a launch has at most 2^32 threads, 8 a point here
   for (long first = 0; first < n; first += kLaunch) {
     const dim3 grid(blocks_for(std::min(n - first, kLaunch), 64));

@@ -81,3 +81,32 @@ def test_a_slab_value_does_not_depend_on_the_points_beside_it(run):
             assert np.array_equal(s.device_values(pts[:n]), many[:n]), n
     finally:
         s.close()
+
+
+def test_threads_with_tables_of_other_lengths():
+    """Two threads, each with its own surface (corrugation functions of 46 and 5 knots, both in LDS), give bit for bit
+    what each gives alone."""
+    import threading
+    import spodvr_amd
+    surfaces = [spodvr_amd.CrpSurface(os.path.join(CRP_DIR, case, "dataset"))
+                for case in ("cu111_srp48", "c3v_impulse_15")]
+    try:
+        points = [_points(s, 1000, 24) for s in surfaces]
+        _note("values of two surfaces, one after the other, then from two threads")
+        alone = [s.device_qd(p) for s, p in zip(surfaces, points)]
+        assert not np.array_equal(*alone)
+        same = [[], []]
+
+        def work(k):
+            for _ in range(50):
+                same[k].append(np.array_equal(surfaces[k].device_qd(points[k]), alone[k]))
+
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert same == [[True] * 50] * 2
+    finally:
+        for s in surfaces:
+            s.close()

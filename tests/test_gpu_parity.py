@@ -30,7 +30,7 @@ CASE_PARAMS = {
 
 def _pair(case, overrides=None, interaction=None):
     """A HIP run and an oracle run of one case. interaction="lds" makes the HIP backend use its LDS-contraction
-    interaction kernel instead of the MFMA one (SPO_HIP_INTERACTION is read when the backend is created). Both
+    interaction kernel instead of the in-place one (SPO_HIP_INTERACTION is read when the backend is created). Both
     runs take the potential grid from the host build, so that these tests compare the propagation alone: the
     device build of the grid agrees with it to rounding (test_gpu_potential.py), but at the strongly repulsive
     points (V of hundreds of hartree) a last-bit difference in V is a phase difference of ~1e-11 after V dt."""
@@ -120,9 +120,9 @@ def test_mixed_precision_t_block_against_fp64_oracle(case):
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("interaction", ["lds", "mfma_staged", "mfma", "buf"])
 def test_interaction_variants_match_oracle(case, precision, interaction):
-    """Every interaction kernel (vector-unit contractions; MFMA contractions with staged phi FFTs, with the fused
-    register phi step (the FP64 default), and with buffer addressing (the complex64 default)) on one full T
-    block."""
+    """Every interaction kernel that SPO_HIP_INTERACTION selects (vector-unit contractions; MFMA contractions with staged
+    phi FFTs, with the fused register phi step, and with buffer addressing) on one full T block; the default, the
+    in-place kernel, is in test_one_t_block_matches_oracle."""
     print(f"case {case} seed 31 interaction {interaction} {precision}", flush=True)
     gpu, cpu = _pair(case, {"Precision": precision}, interaction=interaction)
     _randomise(gpu, cpu, 31)
@@ -185,16 +185,16 @@ def test_two_runs_are_bitwise_identical(precision):
                                            ("hardwall_short", ["zr=256", "zr=512", "xy=32", "xy=64"]),
                                            ("dz", ["xy=8", "xy=16", "xy=32"] + [f"zr=#{k}" for k in range(1, 7)])])
 def test_launch_variants_match_the_default(case, settings, precision):
-    """The launch variants (block sizes, tile widths) against the default variant after a full T block: the same
-    arithmetic up to the compiler's multiply-add contraction, so within the parity bar (FP64 1e-13, complex64 1e-6
-    relative)."""
+    """Some launch variants (block sizes, tile widths, T_Zr radices) against the default variant after a full T block: the
+    same transforms with roundings in another order (FP64 1e-13, complex64 1e-6 relative). test_gpu_variants.py walks
+    every list to its end."""
     import os
     import spodvr_amd
     # dz: the 16 x 16 (x, y) grid of the DZ workload, whose T_xy tiles are 8, 16 or 32 izr wide
     path = cases.write_case("dz", cases.DZ_6D) if case == "dz" else CASE_PARAMS[case]()
     tol = 1e-13 if precision == "fp64" else 1e-6
     if case == "dz_angular" and precision == "mixed":
-        settings = settings + ["interaction=#3"]  # the complex64 default kernel has a fourth (8 x 6 phi radices)
+        settings = settings + ["interaction=#3"]  # behind the three in-place variants: the first buffer kernel
     wave = None
     reference = None
     for setting in ["default"] + settings:

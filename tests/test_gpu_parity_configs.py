@@ -1,11 +1,11 @@
 """HIP backend against the CPU oracle at the two benchmark workloads' own shapes, so that the kernel instantiations
 the benchmark times are the ones checked:
 
-  hardwall_6d  HardWallPES, NZ 128 x NR 32, 8 x 8 (x, y), JMax 10 (6 theta x 22 phi): zr_reg_kernel<128, 32, ...>,
-               xy_reg_kernel<8, 8, ...>, the MFMA interaction kernel with a 22-point phi step;
+  hardwall_6d  HardWallPES, NZ 128 x NR 32, 8 x 8 (x, y), JMax 10 (6 theta x 22 phi): zr_inplace_kernel with
+               ZrStatic<128, 32, ...>, xy_reg_kernel<8, 8, 32>, interaction_kernel_inplace with the 11 x 2 phi step;
   dz_6d        Dai-Light H2/Cu(111), NZ 96 x NR 48, 16 x 16, JMax 24 / MJMax 23 (13 theta x 48 phi), C6v-reduced
-               potential: zr_reg_kernel<96, 48, 3, 16, 8, 12, ...>, xy_reg_kernel<16, 16, {16, 32}>, the MFMA
-               interaction kernel with the 12 x 4 phi step.
+               potential: zr_inplace_kernel with ZrStatic<96, 48, ...>, xy_reg_kernel<16, 16, 32>,
+               interaction_kernel_inplace with the 16 x 3 phi step.
 
 Same measure as the reference's CPU-vs-GPU check (tests/cuda/test_cuda_backend.cpp:94-106): max |a - b| / max |a|
 after one T block (full, half, kinetic only) and after one analysis step from the same seeded wave packet, 1e-12 in

@@ -46,6 +46,94 @@ def test_gradient_matches_oracle():
         net.close()
 
 
+def _batch(rows, seed):
+    rng = np.random.default_rng(seed)
+    return rng.normal(size=(rows, 6)).astype(np.float32), rng.normal(size=rows).astype(np.float32)
+
+
+@pytest.mark.parametrize("batch", [16, 48, 272, 4112])
+def test_gradient_of_batches_that_fill_no_round(batch):
+    """One row tile, fewer tiles than a workgroup has wavefronts, one more than the update's round of 16 tiles, and many
+    rounds and one tile. The bound of test_gradient_matches_oracle, and for the smallest batches one bf16 operand more,
+    rounded the other way (2^-7 of a term that may be most of an entry's few)."""
+    import spodvr_amd
+    _note("gradient, batch", batch)
+    bound = 2e-3 + (2.0 ** -7 if batch < 256 else 0.0)
+    net = spodvr_amd.Mlp(batch)
+    try:
+        p = mlp.initial_parameters(6)
+        net.params = p
+        x, t = _batch(batch, 7)
+        loss, grad = net.gradient(x, t)
+        ref_loss, ref_grad = mlp.loss_and_gradient(p.astype(np.float64), x, t)
+        assert abs(loss - ref_loss) <= (1e-5 if batch >= 256 else 1e-4) * abs(ref_loss)
+        offsets = np.cumsum([0] + [int(np.prod(s)) for s in mlp.SHAPES])
+        for k in range(len(mlp.SHAPES)):
+            a, b = grad[offsets[k]:offsets[k + 1]], ref_grad[offsets[k]:offsets[k + 1]]
+            assert np.max(np.abs(a - b)) <= bound * np.max(np.abs(b)), k
+    finally:
+        net.close()
+
+
+@pytest.mark.parametrize("batch", [48, 272])
+def test_adam_steps(batch):
+    """Six training steps, each against Adam in numpy on the device's own gradient before it (FP32 rounding: 1e-4 of the
+    learning rate, from 1 - beta2^t, and an ulp or two of the parameter); after them the bf16 copies of the weights that
+    the steps kept up to date give bit for bit the gradient of copies made anew from the same parameters."""
+    import spodvr_amd
+    _note("Adam steps, batch", batch)
+    lr, beta1, beta2 = np.float32(1e-3), np.float32(0.9), np.float32(0.999)
+    net, fresh = spodvr_amd.Mlp(batch), spodvr_amd.Mlp(batch)
+    try:
+        net.params = mlp.initial_parameters(8)
+        p = net.params.astype(np.float64)
+        m, v = np.zeros_like(p), np.zeros_like(p)
+        for step in range(1, 7):
+            x, t = _batch(batch, 20 + step)
+            loss, g = net.gradient(x, t)
+            losses = net.train(x, t, steps=1, lr=float(lr))
+            assert abs(losses[0] - loss) <= 1e-6 * loss
+            m = float(beta1) * m + (1.0 - float(beta1)) * g
+            v = float(beta2) * v + (1.0 - float(beta2)) * g.astype(np.float64) ** 2
+            c1, c2 = 1.0 - float(beta1) ** step, 1.0 - float(beta2) ** step
+            p = p - float(lr) * (m / c1) / (np.sqrt(v / c2) + 1e-8)
+            got = net.params
+            assert np.max(np.abs(got - p) - (1e-4 * lr + 2.0 ** -22 * np.abs(p))) <= 0.0, step
+            p = got.astype(np.float64)
+        fresh.params = net.params
+        x, t = _batch(batch, 30)
+        (loss, g), (loss_new, g_new) = net.gradient(x, t), fresh.gradient(x, t)
+        assert loss == loss_new and np.array_equal(g, g_new)
+        assert np.array_equal(net.predict(x), fresh.predict(x))
+    finally:
+        net.close()
+        fresh.close()
+
+
+def test_prediction_of_any_number_of_rows():
+    """Less than a tile, and a tile and one row, against the oracle; more rows than the workgroups of a launch take in one
+    round (32768) and more than one launch takes (2^20) bit for bit as in calls of fewer rows. (Against the oracle a few
+    of that many rows are off by 1e-3: an operand that lies on the edge of two bf16 values is rounded the other way.)"""
+    import spodvr_amd
+    net = spodvr_amd.Mlp(256)
+    try:
+        p = mlp.initial_parameters(9)
+        net.params = p
+        for rows in (1, 15, 17):
+            _note("prediction of", rows, "rows")
+            x, _ = _batch(rows, 40)
+            ref, _ = mlp.forward(p.astype(np.float64), x)
+            assert np.max(np.abs(net.predict(x) - ref)) <= 1e-4 * max(1.0, np.max(np.abs(ref)))
+        for rows, first in ((40001, 0), ((1 << 20) + 17, (1 << 20) - 2000)):
+            _note("prediction of", rows, "rows")
+            x, _ = _batch(rows, 41)
+            y = net.predict(x)
+            for k in range(first, rows, 1000):
+                assert np.array_equal(y[k:k + 1000], net.predict(x[k:k + 1000])), k
+    finally:
+        net.close()
+
+
 def test_training_on_crp_energies_converges():
     import spodvr_amd
     from spodvr_amd import surrogate

@@ -58,6 +58,13 @@ def test_zr_plane_shapes(nz, nr):
     _check(f"zr_{nz}_{nr}", _grid(nz, nr, 4, 2), 100 + nz + nr, blocks=((False, False), (True, True)))
 
 
+# Planes beyond the in-place kernel in FP64: 160 x 64 fits a CU's LDS only without the padding of its rows (the run-time
+# engine on the plane), 176 x 64 does not fit at all (line transforms). In complex64 both are in place.
+@pytest.mark.parametrize("nz,nr", [(160, 64), (176, 64)])
+def test_zr_planes_beyond_the_in_place_kernel(nz, nr):
+    _check(f"zr_{nz}_{nr}", _grid(nz, nr, 4, 2), 100 + nz + nr, blocks=((False, False), (True, True)))
+
+
 # Specular grids (NZSpecular, NR) on both sides of each choice: in one launch, with small radices and with 18, 20 and 22
 # along Z, before the scattering wave's step (up to 5120 points) and beside it; no product of two radices (420), and
 # more points than a CU's LDS holds (360 x 36), which take the line transforms.

@@ -17,7 +17,16 @@ from tests.util import pseudo_random, relative_difference
 pytestmark = pytest.mark.gpu
 
 
+# Grids without compile-time kernels: the run-time-shaped T_Zr in row mode and the (x, y) kernels of other lengths on the
+# row. NZ, NR, NX = NY, Zana.
+RUN_TIME_SHAPES = {"run_time_90_40_10": (90, 40, 10, 7.5), "run_time_66_12_6": (66, 12, 6, 7.1)}
+
+
 def _case_input(case):
+    if case in RUN_TIME_SHAPES:
+        from tests.test_gpu_grid_shapes import _grid
+        nz, nr, nxy, zana = RUN_TIME_SHAPES[case]
+        return cases.write_case(case, _grid(nz, nr, nxy, 4, Zana=zana)), {}
     if case == "dz_angular":
         return cases.write_case("dz_angular", cases.DZ_ANGULAR), {}
     return cases.golden_input(case), cases.golden_overrides(case)
@@ -113,3 +122,19 @@ def test_switch_values_other_than_0_and_1_are_refused():
             os.environ.pop("SPO_HIP_MERGE_HALF_STEPS", None)
         else:
             os.environ["SPO_HIP_MERGE_HALF_STEPS"] = old
+
+
+def test_run_time_shapes_have_an_even_and_an_odd_analysis_row():
+    rows = []
+    for case in RUN_TIME_SHAPES:
+        print(f"case {case}: set-up", flush=True)
+        run = _run(case, "fp64", True)
+        rows.append(run.info.iz_analysis % 2)
+        run.close()
+    assert rows == [0, 1]
+
+
+@pytest.mark.parametrize("case", list(RUN_TIME_SHAPES))
+def test_merged_half_steps_on_run_time_shapes(case):
+    test_fp64_merged_half_steps_match_the_plain_schedule(case)
+    test_complex64_merged_half_steps_keep_the_accuracy(case)

@@ -9,7 +9,11 @@ namespace spo_dev {
 
 // Radices (R1, R2) of the phi lengths that an angular grid takes up to MJMax 31: coprime wherever the length allows
 // it (no twiddles), the smaller one second (a thread holds R2 values of the row, of exp(i A) and of the next exp(i A):
-// 22 points as 2 x 11 in FP64 spilled and took 347 us at the HardWall workload, as 11 x 2 150), one pass up to 8 points.
+// 22 points as 2 x 11 in FP64 took 347 us at the HardWall workload, as 11 x 2 150), one pass up to 8 points. Four
+// wavefronts a SIMD leave a lane 128 registers, and in FP64 the offsets and exp(i A) values that live across the R1 pass
+// do not all fit: the default variants spill 2 registers at 22 points (12 bytes of scratch a lane), 1 at 42 (8), 10 at 44
+// (44), 6 at 48 (28), 1 at 50 (8), 10 at 54 (44) and 74 at 64 (236); none at the other lengths and none in complex64.
+// At 48 points (13 theta, 96 x 48 x 16 x 16) a launch writes 1.04 GB of scratch beside the wave's 4.19 GB.
 #define SPO_PHI_RADICES(X)                                                                                    \
   X(2, 1) X(4, 1) X(6, 1) X(8, 1) X(5, 2) X(4, 3) X(7, 2) X(4, 4) X(9, 2) X(5, 4) X(11, 2) X(8, 3) X(7, 4)      \
   X(10, 3) X(8, 4) X(9, 4) X(8, 5) X(14, 3) X(11, 4) X(16, 3) X(10, 5) X(9, 6) X(8, 7) X(12, 5) X(8, 8)
@@ -24,6 +28,9 @@ namespace spo_dev {
 // Complex64 takes tiles of 16 columns (whole 128-byte lines of a row; at 13 theta x 48 phi 2500 us against 3110 of 8
 // columns), except the shortest rows, where one wavefront's worth of them is enough. A launch of few workgroups
 // (the device holds 4096 of these) takes two wavefronts for the latency (64 x 16 x 4 x 4: 13.5 us against 15.2).
+// 56 points in FP64 stay with interaction_mfma_kernel: at 13 to 15 theta one tile fills a CU, and with the 16 wavefronts
+// that it then takes this kernel spilled 25 registers: 594 us (48 x 24 x 8 x 8, 14 theta) against 546 there, and 2149
+// against 1960 (96 x 48 x 8 x 8).
 template <typename T>
 std::vector<Variant> interaction_inplace_variants(int nphi, int n_theta, long columns) {
   std::vector<Variant> out;
@@ -37,6 +44,7 @@ std::vector<Variant> interaction_inplace_variants(int nphi, int n_theta, long co
       Y(R1, R2, 1, 1) Y(R1, R2, 1, 2)                                                                         \
     } else if constexpr (sizeof(T) == 4) {                                                                    \
       Y(R1, R2, 2, 4) Y(R1, R2, 2, 8) Y(R1, R2, 2, 16)                                                        \
+    } else if constexpr (R1 * R2 == 56) {  /* see above */                                                    \
     } else if constexpr (R1 * R2 <= 22) {                                                                     \
       Y(R1, R2, 1, 1) Y(R1, R2, 1, 2) Y(R1, R2, 1, 4)                                                         \
     } else {                                                                                                  \

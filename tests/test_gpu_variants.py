@@ -68,8 +68,8 @@ def _check(name, params, seed, family, precisions=("fp64", "mixed"), interaction
 
 
 # Angular bases of every phi length that these grids take up to MJMax 31 (2, 4, ... 24, 28, 30, 32, 36, 40, 42, 44, 48,
-# 56, 60 and 64 points), an (izr) count that fills no tile, with the MFMA and buffer kernels' own lists where they have
-# one.
+# 56, 60 and 64 points; 56 in FP64 has MFMA kernels alone), an (izr) count that fills no tile, with the MFMA and buffer
+# kernels' own lists where they have one.
 @pytest.mark.parametrize("jmax,mjmax,homonuclear", [
     (0, 0, True), (1, 1, False), (2, 2, True), (3, 3, False), (4, 4, True), (5, 5, False), (6, 6, True), (7, 7, False),
     (8, 8, True), (9, 9, False), (10, 10, True), (11, 11, False), (12, 12, True), (14, 14, True), (15, 15, False),

@@ -314,7 +314,9 @@ __global__ __launch_bounds__(64 * kProjectionWaves) void projection_kernel(cx<T>
 // Analysis. One workgroup per (v, irotana): overlap over r with phi_vj(r) dR and the momentum shift, (x, y) FFT
 // (sign -, scale 1), pick the analysed diffraction slots (src/analysis/balint_kurti.cpp:52-72). Every coefficient is
 // written. spec not NULL: the initial state's are taken from the specular wave at the fixed analysis surface instead
-// (:74-82), by the workgroup whose coefficient it is; phi_in(ir, v) the initial state's radial functions.
+// (:74-82), by the workgroup whose coefficient it is; phi_in(ir, v) the initial state's radial functions. Without a
+// launch bound the compiler allows for 1024 threads: 128 registers, and 328 bytes of scratch a lane. 23 us at HardWall
+// and 60 at DZ, once an analysis step.
 template <typename T>
 __global__ void bk_scattering_kernel(const cx<T>* psi, Shape s, int iz_ana, int n_rot_ana, int n_dif,
                                      int n_states, const int* rot_index, const int* slots, const double* weights,

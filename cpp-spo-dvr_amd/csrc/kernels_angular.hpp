@@ -18,6 +18,11 @@
 //    exp(i A) are set up once.
 // 3. DVR -> FBR, x rot(dt/2), stored straight to HBM. The factor depends on J and r alone: the table holds one row
 //    per distinct row of the caller's (irot, ir) table (rows of one J come out the same), short enough for the L1.
+//
+// Bound by latency: the phases of a tile wait for each other. At DZ (13 theta x 48 phi, two 82 KB tiles a CU) wavefronts
+// wait in 51 % of their cycles in FP64 and 46 in complex64, with the vector units busy 32 and 52 %, the matrix cores 20
+// and 20, LDS 19 and 24: 3.95 and 2.42 ms a launch for 9.33 and 4.67 GB. At 128 registers a lane some FP64 lengths keep
+// values in scratch too (variants_angular.hpp).
 #pragma once
 
 #include "fft_ct.hpp"

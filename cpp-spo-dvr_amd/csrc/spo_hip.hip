@@ -457,9 +457,9 @@ struct State final : spo_hip_backend {
   const void* v_fn = nullptr;
   bool zr_fused = false;
 
-  // The T_Zr factors in the order of zr_inplace_kernel's places (order_zr_factors, for the variant in use).
-  Buffer zr_full_p, zr_half_p, zr_full_p_lo, zr_half_p_lo;
-  void order_zr_factors(const std::vector<double>& full, const std::vector<double>& half, const spo_dev::ZrShape& order);
+  // The T_Zr factors (and complex64 remainders), natural or in the order of zr_inplace_kernel's places, for the kernel in
+  // use.
+  void upload_zr_factors(const std::vector<double>& full, const std::vector<double>& half, const spo_dev::ZrShape* order);
 
   Buffer ana_row;  // the analysis row of the scattering wave at the analysis time (merged half steps)
 
@@ -504,29 +504,29 @@ void State<T>::run_zr(const Variant& v, bool half, cx<T>* row_out, int row) {
   const T* ez = plan_z->tw_eps();
   const T* er = plan_r->tw_eps();
   spo_dev::ZrShape shape = v.zr;
-  const cx<T>* zr = (half ? zr_half_p : zr_full_p).as<cx<T>>();
-  const cx<T>* fl = (half ? zr_half_p_lo : zr_full_p_lo).as<cx<T>>();
+  const cx<T>* zr = (half ? zr_half : zr_full).as<cx<T>>();
+  const cx<T>* fl = (half ? zr_half_lo : zr_full_lo).as<cx<T>>();
   void* args[] = {&ps, &shape, const_cast<cx<T>**>(&tz), const_cast<cx<T>**>(&tr), const_cast<cx<T>**>(&zr),
                   const_cast<T**>(&ez), const_cast<T**>(&er), const_cast<cx<T>**>(&fl), &row_out, &row};
   launch(v.fn, s.n_rot * s.n_xy, v.threads, v.lds, stream, args);
 }
 
 template <typename T>
-void State<T>::order_zr_factors(const std::vector<double>& full, const std::vector<double>& half,
-                                const spo_dev::ZrShape& order) {
-  std::vector<double> f(full.size()), h(half.size());
-  for (int iz = 0; iz < s.nz; ++iz)
+void State<T>::upload_zr_factors(const std::vector<double>& full, const std::vector<double>& half,
+                                 const spo_dev::ZrShape* order) {
+  std::vector<double> f(full), h(half);
+  for (int iz = 0; order && iz < s.nz; ++iz)
     for (int ir = 0; ir < s.nr; ++ir) {
-      const std::size_t to = 2 * (ir + std::size_t(s.nr) * iz), from = 2 * spo_dev::zr_factor_order(order, iz, ir);
+      const std::size_t to = 2 * (ir + std::size_t(s.nr) * iz), from = 2 * spo_dev::zr_factor_order(*order, iz, ir);
       for (int c = 0; c < 2; ++c) {
         f[to + c] = full[from + c];
         h[to + c] = half[from + c];
       }
     }
-  zr_full_p = upload_complex<T>(f.data(), s.n_zr);
-  zr_full_p_lo = factor_lo<T>(f.data(), s.n_zr);
-  zr_half_p = upload_complex<T>(h.data(), s.n_zr);
-  zr_half_p_lo = factor_lo<T>(h.data(), s.n_zr);
+  zr_full = upload_complex<T>(f.data(), s.n_zr);
+  zr_full_lo = factor_lo<T>(f.data(), s.n_zr);
+  zr_half = upload_complex<T>(h.data(), s.n_zr);
+  zr_half_lo = factor_lo<T>(h.data(), s.n_zr);
 }
 
 template <typename T>
@@ -1136,15 +1136,9 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
     for (double& x : v) x = x * f1 * f2;
     return v;
   };
-  std::vector<double> zr_full_values, zr_half_values;
+  const std::vector<double> zr_full_values = fold(t->zr_full, s.n_zr, zr_f, zr_b);
+  const std::vector<double> zr_half_values = fold(t->zr_half, s.n_zr, zr_f, zr_b);
   {
-    const auto zf = fold(t->zr_full, s.n_zr, zr_f, zr_b), zh = fold(t->zr_half, s.n_zr, zr_f, zr_b);
-    b->zr_full = upload_complex<T>(zf.data(), s.n_zr);
-    b->zr_full_lo = factor_lo<T>(zf.data(), s.n_zr);
-    b->zr_half = upload_complex<T>(zh.data(), s.n_zr);
-    b->zr_half_lo = factor_lo<T>(zh.data(), s.n_zr);
-    zr_full_values = zf;
-    zr_half_values = zh;
     const auto sf = fold(t->specular_full, std::size_t(s.nr) * s.nzsp, zr_f, sp_b);
     const auto sh = fold(t->specular_half, std::size_t(s.nr) * s.nzsp, zr_f, sp_b);
     b->spec_lds = spo_dev::zr_plane_lds<double>(s.nzsp, s.nr);
@@ -1269,12 +1263,12 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
   if (spo_dev::zr_plane_lds<T>(s.nz, s.nr) <= lds_limit) b->zr_variants = spo_dev::zr_variants<T>(s.nz, s.nr);
   if (!b->zr_variants.empty()) {
     for (const Variant& v : b->zr_variants) set_lds(v.fn, lds_limit);  // one kernel serves planes of many sizes
-    b->order_zr_factors(zr_full_values, zr_half_values, b->zr_variants[0].zr);
   } else if (std::size_t(s.n_zr) * cT <= lds_limit) {
     b->zr_fused = true;
     b->zr_lds = std::size_t(s.n_zr) * cT;
     set_lds(reinterpret_cast<const void*>(spo_dev::zr_plane_kernel<T>), b->zr_lds);
   }
+  b->upload_zr_factors(zr_full_values, zr_half_values, b->zr_variants.empty() ? nullptr : &b->zr_variants[0].zr);
   // T_xy.
   for (const Variant& v : spo_dev::xy_reg_variants<T>(s.nx, s.ny))
     if (v.lds <= lds_limit) b->xy_variants.push_back(v);
@@ -1466,7 +1460,7 @@ std::unique_ptr<spo_hip_backend> create_state(const spo_hip_shape* shape, const 
   HIP_CHECK(hipStreamSynchronize(b->stream));
   b->tune();
   if (b->zr_pick != 0)
-    b->order_zr_factors(zr_full_values, zr_half_values, b->zr_variants[b->zr_pick].zr);
+    b->upload_zr_factors(zr_full_values, zr_half_values, &b->zr_variants[b->zr_pick].zr);
   return b;
 }
 
